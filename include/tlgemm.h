@@ -163,11 +163,11 @@ const char *tlg_group_kernel(void);
  * library's split reduction. */
 int tlg_gemv_status(void);
 /* Tuning hook: pin the tile configuration of grouped launches (an index of
- * the kernel's tile table; -1 = automatic: 64x64 tiles when a launch has at
- * least 3 x 256 of them, else 64x32 tiles whose wave pairs split each stage). */
+ * the kernel's tile table; -1 = automatic: the largest of 128x128, 128x64,
+ * 64x64, 64x32 and 32x32 tiles that gives a launch enough work items). */
 int tlg_tune_group(int cfg);
-/* Tuning hook: the automatic policy itself -- candidate tile configs (up to
- * 3, first that yields min_waves x 256 work items wins, else the last; ncands
+/* Tuning hook: a policy in place of the automatic one -- candidate tile configs
+ * (up to 3, first that yields min_waves x 256 work items wins, else the last; ncands
  * 0 keeps the list), min_waves (<= 0 keeps it) and the target reduction
  * steps per split work item (0 keeps it).  Applies to later launches. */
 int tlg_tune_group_policy(const int *cands, int ncands, double min_waves, int rtarget);
@@ -179,12 +179,10 @@ int tlg_tune_group_policy(const int *cands, int ncands, double min_waves, int rt
 int tlg_tune_group_split(int rtarget);
 /* Tuning hook: the tile shape of the MoE expert launches (tlg_dev_moe_*):
  * cfg -1 = automatic (64x64 tiles of 16-step stages when a launch has about
- * 3 x 256 of them, else 64x32, else 32x32), or 3 (64x64), 18 (64x64, 16-step
- * stages), 14 (64x32), 15 (32x32), 22 (16-wave 64x64, whose waves split each
- * 64-step stage four ways) pinned;
- * sched 1 = each stage's fragment reads issued before its MFMAs, 2 = that
- * order with the outputs written by streaming stores, 0 = the compiler's
- * order, -1 = automatic (2 for the fused SwiGLU launches of dense rows, 1 for
+ * 320 of them, else 64x32, else 32x32), or 3 (64x64), 18 (64x64, wave pairs
+ * each taking half of a 32-step stage), 14 (64x32), 15 (32x32), 22 (8-wave
+ * 64x64, whose waves split each 64-step stage four ways) pinned;
+ * sched 0 or 1 = plain stores, 2 = streaming stores, -1 = automatic (2 for the fused SwiGLU launches of dense rows, 1 for
  * MoE launches).  Applies to later launches. */
 int tlg_tune_expert(int cfg, int sched);
 

@@ -1,0 +1,118 @@
+"""The tile kernels' arithmetic: fp32 operands as three bf16 pieces each, six
+products of them on the matrix cores.  Error against fp64, operands that have
+no such split (infinities, NaN, magnitudes past bf16's largest), and the
+sizes where a tile, a stage or a chunk ends."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _torch():
+    import torch
+    return torch
+
+
+@pytest.fixture(scope="module")
+def lib():
+    import tlgemm
+    _torch().cuda.init()
+    L = tlgemm.load()
+    L.check(L.tlg_init(0), "tlg_init")
+    return L
+
+
+def run(lib, op, X, W, dY, grouped):
+    """The primitive on device copies (accumulating ones from zero), as numpy."""
+    torch = _torch()
+    M, K, N = X.shape[0], X.shape[1], W.shape[1]
+    x, w, dy = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (X, W, dY))
+    shape = {"mm": (M, N), "mm_bt": (M, K), "mm_atb": (K, N)}[op]
+    out = torch.zeros(shape, device="cuda")
+    a, b = {"mm": (x, w), "mm_bt": (dy, w), "mm_atb": (x, dy)}[op]
+    st = torch.cuda.current_stream().cuda_stream
+    if grouped:
+        lib.group([dict(op=op, beta=0 if op == "mm" else 1, C=out.data_ptr(), M=M, K=K, N=N, A=[a.data_ptr()],
+                        B=[b.data_ptr()])], st)
+    else:
+        {"mm": lib.mm, "mm_bt": lib.mm_bt, "mm_atb": lib.mm_atb}[op](out.data_ptr(), a.data_ptr(), b.data_ptr(), M, K,
+                                                                    N, st)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+def want(op, X, W, dY):
+    X, W, dY = (a.astype(np.float64) for a in (X, W, dY))
+    with np.errstate(all="ignore"):
+        return {"mm": lambda: X @ W, "mm_bt": lambda: dY @ W.T, "mm_atb": lambda: X.T @ dY}[op]()
+
+
+def reduction(op, M, K, N):
+    return {"mm": K, "mm_bt": N, "mm_atb": M}[op]
+
+
+# (M, K, N): a tile, stage or chunk ends one short, exactly, or one past
+EDGES = [(9, 16, 16), (32, 32, 32), (33, 20, 68), (64, 15, 64), (65, 17, 63), (127, 48, 129), (128, 128, 128),
+         (257, 131, 259), (300, 64, 36), (513, 4, 72), (1024, 512, 192), (2050, 72, 516)]
+
+
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+@pytest.mark.parametrize("shape", EDGES, ids=str)
+def test_error_against_fp64(lib, op, shape):
+    """Each product is exact to 2^-25 and each 16-step MFMA adds one rounding
+    of the running sum (2^-24): over R steps the error's 2-norm stays under
+    2^-24 (1 + sqrt(R / 16)) times the result's for random signs, with room
+    for the rounding inside an MFMA (x 4)."""
+    M, K, N = shape
+    r = np.random.default_rng(M * 7 + K)
+    X = r.standard_normal((M, K), dtype=np.float32)
+    W = (0.02 * r.standard_normal((K, N))).astype(np.float32)
+    dY = (0.01 * r.standard_normal((M, N))).astype(np.float32)
+    ref = want(op, X, W, dY)
+    R = reduction(op, M, K, N)
+    tol = 4 * 2.0 ** -24 * (1 + np.sqrt(R / 16))
+    for grouped in (False, True):
+        if grouped and (M % 4 and op == "mm_atb" or K % 4 or N % 4):
+            continue
+        got = run(lib, op, X, W, dY, grouped)
+        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert err <= tol, (op, shape, grouped, err, tol)
+
+
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+@pytest.mark.parametrize("grouped", [False, True])
+@pytest.mark.parametrize("shape", [(40, 36, 52), (200, 132, 260)], ids=str)
+def test_operands_without_a_split(lib, op, grouped, shape):
+    """Infinities, NaN and values that round to bf16's infinity give what fp32
+    sums give, and leave the outputs they do not enter alone."""
+    M, K, N = shape
+    r = np.random.default_rng(3)
+    X = r.standard_normal((M, K), dtype=np.float32)
+    W = r.standard_normal((K, N), dtype=np.float32)
+    dY = r.standard_normal((M, N), dtype=np.float32)
+    a, b = {"mm": (X, W), "mm_bt": (dY, W), "mm_atb": (X, dY)}[op]
+    a[3, 5], a[17, 2], a[8, 9] = np.inf, np.nan, np.float32(3.4e38)
+    b[1, 7], b[6, 11] = -np.inf, np.float32(-3.4e38)
+    if op == "mm_atb":
+        a[:, 20] = 0.0                               # 0 x inf
+    got, ref = run(lib, op, X, W, dY, grouped), want(op, X, W, dY)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(got[inf], np.sign(ref[inf]) * np.inf)
+    # elsewhere each of R roundings is at most 2^-24 of the terms' absolute sum
+    # (where that sum is in range: a partial sum past it is infinite in fp32)
+    terms = want(op, *(np.abs(np.where(np.isfinite(t), t, 0.0)) for t in (X, W, dY)))
+    fine = np.isfinite(ref) & (terms < 3.3e38)
+    assert fine.any()
+    assert (np.abs(got[fine] - ref[fine]) <= reduction(op, M, K, N) * 2.0 ** -24 * terms[fine]).all()
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-18, 1e18])
+def test_magnitudes(lib, scale):
+    """The pieces keep fp32's exponent range: tiny and huge operands are as
+    exact as ordinary ones while the products are in range."""
+    r = np.random.default_rng(5)
+    X = (scale * r.standard_normal((96, 80))).astype(np.float32)
+    W = (r.standard_normal((80, 112)) / (scale if scale > 1 else 1)).astype(np.float32)
+    got, ref = run(lib, "mm", X, W, W[:1], False), want("mm", X, W, W[:1])
+    assert np.linalg.norm(got - ref) <= 4 * 2.0 ** -24 * (1 + np.sqrt(5)) * np.linalg.norm(ref)

@@ -1,650 +1,10 @@
-// tlg_gemm.hip -- fp32 MFMA GEMM kernels for gfx950 behind mm / mm_bt / mm_atb.
-//
-// One tile routine serves the three reference primitives (tinylm.c:438-537):
-//
-//   mm      Y  = X  W      C(i,j) = sum_r X[i][r]  W[r][j]     NN
-//   mm_bt   dX += dY W^T   C(i,j) = sum_r dY[i][r] W[j][r]     NT
-//   mm_atb  dW += X^T dY   C(i,j) = sum_r X[r][i]  dY[r][j]    TN
-//
-// Each operand is either contiguous along the reduction index r ("RC") or
-// along its output index ("OC").  A workgroup of 4 wave64s owns a BM x BN
-// tile of C; each wave owns a (BM/WGM) x (BN/WGN) sub-tile built from 32x32
-// v_mfma_f32_32x32x2_f32 blocks.  Operand tiles of BK reduction steps are
-// staged global -> registers -> LDS: loads run two stages ahead of the MFMAs
-// (two register stages), LDS is double buffered, one barrier per stage.
-//
-// LDS layouts (both give conflict-free fragment reads):
-//   RC operand: [outer][BK+4]  -- a lane reads BK/2 consecutive r of one row
-//                                 with ds_read_b128; the +4 pad rotates rows
-//                                 across banks.
-//   OC operand: [BK][outer+4]  -- 32 lanes read 32 consecutive outer indices
-//                                 of one r row (ds_read_b32).
-//
-// Reduction order inside a tile: MFMA lanes 0-31 supply r in the first half
-// of each BK step and lanes 32-63 the second half, so a lane's BK/2 values
-// are contiguous in an RC tile.  Any fixed bijection of r is a valid MFMA
-// k-order; the result differs from the reference's sequential chain only by
-// fp32 rounding (parity bar: max|err| / mean|ref| <= 1e-4).
-//
-// Split reduction: when output tiles are too few to fill 256 CUs (mm_atb's
-// dW is small, its reduction long), the r range is split over `splits`
-// workgroups.  Each writes its partial sum as a plain Mo x No matrix into a
-// workspace; a later kernel adds the partials to C in split order
-// (deterministic) and applies beta.  Nothing crosses workgroups inside a
-// kernel, so no device-scope fence is needed: on gfx950 such a fence writes
-// back and invalidates the XCD's L2, which costs every co-resident workgroup
-// its cached operands.
-//
-// Grouped launches (tlg_dev_gemm_group): one kernel runs a list of problems
-// of any of the three kinds -- the GEMMs a caller issues back to back with
-// no other work in between -- plus the deferred split reductions of the
-// previous grouped launch.  The kernel boundary between the two launches is
-// what makes the partials visible, so a split costs no extra launch.
-#include "tlg_internal.h"
+// tlg_gemm.hip -- host side of the GEMMs behind mm / mm_bt / mm_atb: shapes,
+// plans and launches of the tile kernels (tlg_tile.h, tlg_tiles.hip), grouped
+// and expert-batched launches, the fills and the measurement probes.
+#include "tlg_tile.h"
 #include <mutex>
 #include <stdio.h>
 #include <string.h>
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-enum { RC = 0, OC = 1 };
-
-// Stage one operand tile into registers.  OUTER = tile extent along the
-// operand's output index, rows/cols beyond `oext` or r beyond `rend` read 0.
-//
-// Two forms serve the expert GEMMs of the MoE layer (float4 path only):
-//   G   gathered rows: the operand's memory row of tile row x is rs[q], read
-//       from a row map -- once per tile for an RC operand (rows(): the rows
-//       are output rows), once per stage for an OC operand (prep(): the rows
-//       are reduction steps; prep runs a full prefetch round ahead of the
-//       load that uses it, so waiting for the map never waits for the
-//       operand loads issued after it).
-//   PB  paired columns (OC only): tile columns [0, OUTER/2) come from P and
-//       [OUTER/2, OUTER) from P2, both at columns o0 + [0, OUTER/2).
-// Sixteen zero bytes in global memory: with ZP a chunk outside the operand
-// is loaded from here instead of being zeroed after its load, so nothing
-// between a stage's loads and its LDS store waits on the loaded values.
-__device__ __attribute__((aligned(16))) float g_zero_chunk[4] = {0.f, 0.f, 0.f, 0.f};
-
-template <int LAY, int OUTER, int BK, bool VEC, int NT, bool G = false, bool PB = false, bool ZP = false>
-struct TileLoader {
-    static constexpr int NCH = OUTER * BK / 4;        // float4 chunks per tile
-    static constexpr int PER = NCH / NT;              // chunks per thread
-    static constexpr int HALF = OUTER / 2;
-    static_assert(NCH % NT == 0, "tile must split evenly over the workgroup's threads");
-    static_assert(!PB || (LAY == OC && HALF % 4 == 0), "paired columns: OC tiles");
-    static_assert(!(G || PB) || VEC, "gathered / paired tiles load float4");
-    f32x4 v[PER];
-    unsigned ok;                                      // bit q: chunk q in range
-    int rs[G ? PER : 1];                              // gathered memory rows
-
-    __device__ __forceinline__ void rows(const int *__restrict__ map, int o0, int oext, int tid)
-    {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = tid + NT * q;
-            rs[q] = map[min(o0 + e / (BK / 4), oext - 1)];
-        }
-    }
-    __device__ __forceinline__ void prep(const int *__restrict__ map, int r0, int rend, int tid)
-    {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = tid + NT * q;
-            rs[q] = map[min(r0 + e / (OUTER / 4), rend - 1)];
-        }
-    }
-
-    // The float4 path issues every load unconditionally from a clamped, in-
-    // bounds address and zeroes out-of-range chunks at store time: branch-free
-    // loads let the compiler count outstanding loads exactly, so waiting for
-    // one stage does not wait for the stages prefetched after it.
-    __device__ __forceinline__ void load(const float *__restrict__ P, int ld, int o0, int oext,
-                                         int r0, int rend, int tid, const float *__restrict__ P2 = nullptr)
-    {
-        ok = 0;
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = tid + NT * q;
-            int o, r;
-            if (LAY == RC) { o = e / (BK / 4); r = (e % (BK / 4)) * 4; }
-            else           { r = e / (OUTER / 4); o = (e % (OUTER / 4)) * 4; }
-            const float *Pq = P;
-            if (PB && o >= HALF) { o -= HALF; Pq = P2; }
-            const int go = o0 + o, gr = r0 + r;
-            f32x4 x = {0.f, 0.f, 0.f, 0.f};
-            if (VEC) {
-                const bool in = go < oext && gr < rend;
-                if (!ZP) ok |= in ? (1u << q) : 0u;
-                // RC: rows clamp to oext-1, r to rend-4; OC: columns clamp to
-                // oext-4, rows to rend-1 (rend, oext are multiples of 4 here)
-                const int gc = (LAY == RC) ? min(go, oext - 1) : min(go, oext - 4);
-                const int rc = (LAY == RC) ? min(gr, rend - 4) : min(gr, rend - 1);
-                const size_t row = G ? (size_t)rs[q] : (size_t)((LAY == RC) ? gc : rc);
-                const float *p = (LAY == RC) ? Pq + row * ld + rc : Pq + row * ld + gc;
-                if (ZP) p = in ? p : g_zero_chunk;
-                x = *reinterpret_cast<const f32x4 *>(p);
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int oo = (LAY == RC) ? go : go + c;
-                    const int rr = (LAY == RC) ? gr + c : gr;
-                    if (oo < oext && rr < rend)
-                        x[c] = (LAY == RC) ? P[(size_t)oo * ld + rr] : P[(size_t)rr * ld + oo];
-                }
-            }
-            v[q] = x;
-        }
-    }
-
-    __device__ __forceinline__ void store(float *__restrict__ L, int tid) const
-    {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int e = tid + NT * q;
-            int o, r;
-            if (LAY == RC) { o = e / (BK / 4); r = (e % (BK / 4)) * 4; }
-            else           { r = e / (OUTER / 4); o = (e % (OUTER / 4)) * 4; }
-            const int off = (LAY == RC) ? o * (BK + 4) + r : r * (OUTER + 4) + o;
-            const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-            *reinterpret_cast<f32x4 *>(L + off) = (!VEC || ZP || ((ok >> q) & 1u)) ? v[q] : z;
-        }
-    }
-};
-
-template <int LAY, int OUTER, int BK>
-struct LdsSize {
-    static constexpr int value = (LAY == RC) ? OUTER * (BK + 4) : BK * (OUTER + 4);
-};
-
-// Fragment of one 32-wide MFMA block: the RW/2 r-values lane (o, h) feeds,
-// from the RW reduction steps [r_base, r_base + RW) of a BK-step stage.
-template <int LAY, int OUTER, int BK, int RW>
-__device__ __forceinline__ void read_frag(const float *__restrict__ L, int o_base, int r_base, int lane,
-                                          float (&f)[RW / 2])
-{
-    const int o = o_base + (lane & 31), h = lane >> 5;
-    if (LAY == RC) {
-        const float *p = L + o * (BK + 4) + r_base + h * (RW / 2);
-#pragma unroll
-        for (int s = 0; s < RW / 2; s += 4) {
-            const f32x4 x = *reinterpret_cast<const f32x4 *>(p + s);
-            f[s] = x[0]; f[s + 1] = x[1]; f[s + 2] = x[2]; f[s + 3] = x[3];
-        }
-    } else {
-#pragma unroll
-        for (int s = 0; s < RW / 2; s++) f[s] = L[(r_base + h * (RW / 2) + s) * (OUTER + 4) + o];
-    }
-}
-
-// Tile geometry.  The 4 waves of a workgroup form a WGM x WGN grid over the
-// BM x BN tile and WK groups along the reduction: with WK > 1 every wave
-// computes its (BM/WGM) x (BN/WGN) sub-tile over RW = BK/WK of each stage's
-// reduction steps, and the WK partial sub-tiles are summed through LDS in
-// fixed order at the end.  WK > 1 gives small tiles several independent MFMA
-// accumulator chains per wave instead of one dependent chain.
-template <int BM_, int BN_, int BK_, int WGM_, int WK_, int NR_ = 2, int NCH_ = 0, int NW_ = 4>
-struct Tile {
-    static constexpr int BM = BM_, BN = BN_, BK = BK_, WGM = WGM_, WK = WK_, NR = NR_;
-    // instruction order of a stage (sched_step): 0 = the compiler's; Sched<>
-    // below selects the others
-    static constexpr int SCH = 0;
-    static constexpr int NW = NW_, THREADS = 64 * NW_;      // waves / threads per workgroup
-    static constexpr int WGN = NW / (WGM * WK);
-    static constexpr int WM = BM / WGM, WN = BN / WGN, FM = WM / 32, FN = WN / 32;
-    static constexpr int RW = BK / WK;
-    // accumulator chains per 32x32 block (the reduction steps of a block
-    // alternate between its NCH chains, summed in fixed order at the store);
-    // measured on MI355X: one chain is as fast and keeps occupancy higher
-    static constexpr int NCH = NCH_ ? NCH_ : 1;
-    static_assert(WGM * WGN * WK == NW && FM >= 1 && FN >= 1, "NW waves, 32x32 blocks");
-    static_assert(RW >= 8 && RW % 8 == 0, "a wave takes a multiple of 8 reduction steps per stage");
-    static constexpr int TILE = BM * BN;
-    template <int LA, int LB>
-    static constexpr int stage_lds() { return 2 * (LdsSize<LA, BM, BK>::value + LdsSize<LB, BN, BK>::value); }
-    static constexpr int red_lds() { return WK > 1 ? WK * TILE : 0; }
-    static constexpr int mx(int a, int b) { return a > b ? a : b; }
-    template <int LA, int LB>
-    static constexpr int lds() { return mx(stage_lds<LA, LB>(), red_lds()); }
-    static constexpr int lds_max() { return mx(mx(lds<RC, OC>(), lds<RC, RC>()), lds<OC, OC>()); }
-    __device__ static int wave() { return threadIdx.x >> 6; }
-    __device__ static int wk() { return wave() / (WGM * WGN); }
-    __device__ static int wm() { return (wave() % (WGM * WGN)) / WGN; }
-    __device__ static int wn() { return (wave() % (WGM * WGN)) % WGN; }
-};
-
-// Instruction order inside one stage's scheduling region (between two
-// barriers).  Left to itself the scheduler interleaves each fragment read
-// with the MFMA pair that consumes it, to save registers, so at one wave
-// per SIMD every MFMA pair waits out a full LDS round trip; the explicit
-// orders issue all of a stage's fragment reads first (the MFMAs then wait
-// only for the oldest ones), optionally behind the prefetch loads.
-template <class T>
-__device__ __forceinline__ void sched_step()
-{
-    constexpr int VMEM_RD = 0x020, DS_RD = 0x100, DS_WR = 0x200, MFMA = 0x008;
-    if constexpr ((T::SCH & 3) == 1) {
-        __builtin_amdgcn_sched_group_barrier(DS_RD, 64, 0);
-        __builtin_amdgcn_sched_group_barrier(MFMA, 64, 0);
-        __builtin_amdgcn_sched_group_barrier(DS_WR, 32, 0);
-    } else if constexpr ((T::SCH & 3) == 2) {
-        __builtin_amdgcn_sched_group_barrier(VMEM_RD, 32, 0);
-        __builtin_amdgcn_sched_group_barrier(DS_RD, 64, 0);
-        __builtin_amdgcn_sched_group_barrier(MFMA, 64, 0);
-        __builtin_amdgcn_sched_group_barrier(DS_WR, 32, 0);
-    }
-}
-
-// A tile shape with an explicit instruction order per stage: 1 = every
-// fragment read of the stage issued before its first MFMA; 2 = the prefetch
-// loads first, then the fragment reads, then the MFMAs.  + 4: the tile's
-// outputs leave with nontemporal (streaming) stores.
-template <class T, int S>
-struct Sched : T {
-    static constexpr int SCH = S;
-};
-
-// acc += A(i0.., r) B(r, j0..) over r in [rbeg, rend).  A tile's loads run
-// NR stages ahead through NR register sets; LDS is double buffered.
-// GA: A's rows go through the row map `amap` (RC A: amap[i0 + x] for tile
-// row x; OC A: amap[r]).  PB: B is the column pair (B, B2) of TileLoader.
-template <class T, int LA, int LB, bool VEC, bool GA = false, bool PB = false>
-__device__ __forceinline__ void tile_accumulate(float *__restrict__ smem, const float *__restrict__ A,
-                                                const float *__restrict__ B, int lda, int ldb,
-                                                int i0, int j0, int Mo, int No, int rbeg, int rend,
-                                                f32x16 (&acc)[T::FM][T::FN][T::NCH],
-                                                const int *__restrict__ amap = nullptr,
-                                                const float *__restrict__ B2 = nullptr)
-{
-    constexpr int BM = T::BM, BN = T::BN, BK = T::BK, RW = T::RW;
-    constexpr int SA = LdsSize<LA, BM, BK>::value, SB = LdsSize<LB, BN, BK>::value;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wm = T::wm(), wn = T::wn(), rb = T::wk() * RW;
-    const int nsteps = (rend - rbeg + BK - 1) / BK;
-    if (nsteps <= 0) return;
-
-    // Every prefetch is issued unconditionally: a stage past the end re-reads
-    // the last stage's (in-bounds) addresses and is never stored.  Loads under
-    // a branch would leave the compiler unsure how many are outstanding where
-    // the paths meet, and it would then wait for all of them, the prefetch
-    // included, before every LDS store.
-    auto stage_r = [&](int st) { return rbeg + min(st, nsteps - 1) * BK; };
-    constexpr bool ZP = T::SCH > 0;
-    TileLoader<LA, BM, BK, VEC, T::THREADS, GA, false, ZP> la0, la1, la2;
-    TileLoader<LB, BN, BK, VEC, T::THREADS, false, PB, ZP> lb0, lb1, lb2;
-    if constexpr (GA && LA == RC) {
-        la0.rows(amap, i0, Mo, tid);
-        la1.rows(amap, i0, Mo, tid);
-        if constexpr (T::NR > 2) la2.rows(amap, i0, Mo, tid);
-    }
-    if constexpr (GA && LA == OC) {
-        la0.prep(amap, rbeg, rend, tid);
-        la1.prep(amap, stage_r(1), rend, tid);
-        if constexpr (T::NR > 2) la2.prep(amap, stage_r(2), rend, tid);
-    }
-    // an OC gather re-arms each register set's row map for the stage it
-    // loads next, NR stages on
-    auto reprep = [&](auto &l, int st) {
-        if constexpr (GA && LA == OC) l.prep(amap, stage_r(st), rend, tid);
-    };
-    la0.load(A, lda, i0, Mo, rbeg, rend, tid);
-    reprep(la0, T::NR);
-    lb0.load(B, ldb, j0, No, rbeg, rend, tid, B2);
-    la1.load(A, lda, i0, Mo, stage_r(1), rend, tid);
-    reprep(la1, 1 + T::NR);
-    lb1.load(B, ldb, j0, No, stage_r(1), rend, tid, B2);
-    if constexpr (T::NR > 2) {
-        la2.load(A, lda, i0, Mo, stage_r(2), rend, tid);
-        reprep(la2, 2 + T::NR);
-        lb2.load(B, ldb, j0, No, stage_r(2), rend, tid, B2);
-    }
-    la0.store(smem, tid);
-    lb0.store(smem + SA, tid);
-    __syncthreads();
-
-    auto compute = [&](const float *As, const float *Bs) {
-        float fa[T::FM][RW / 2], fb[T::FN][RW / 2];
-#pragma unroll
-        for (int a = 0; a < T::FM; a++) read_frag<LA, BM, BK, RW>(As, wm * T::WM + a * 32, rb, lane, fa[a]);
-#pragma unroll
-        for (int b = 0; b < T::FN; b++) read_frag<LB, BN, BK, RW>(Bs, wn * T::WN + b * 32, rb, lane, fb[b]);
-#pragma unroll
-        for (int s = 0; s < RW / 2; s++)
-#pragma unroll
-            for (int a = 0; a < T::FM; a++)
-#pragma unroll
-                for (int b = 0; b < T::FN; b++)
-                    acc[a][b][s % T::NCH] =
-                        __builtin_amdgcn_mfma_f32_32x32x2f32(fa[a][s], fb[b][s], acc[a][b][s % T::NCH], 0, 0, 0);
-    };
-
-    // Stage st lives in LDS buffer st&1 and, before that, in register set
-    // st % NR.  Step st prefetches stage st+NR into the set stage st came
-    // from, computes stage st, then moves stage st+1 from its register set
-    // into the other LDS buffer.  NR = 3 keeps loads three stages ahead.
-    //
-    // Two loop forms, chosen by measurement on MI355X (m3 GEMM set 1.544 ->
-    // 1.51 ms, nano 0.130 -> 0.120 ms, m8 unchanged):
-    // * WK > 1 (the waves split each stage): whole rounds of NR steps with no
-    //   branch inside, the store of stage st+1 unconditional (past the last
-    //   stage it stores the clamped re-read, which nothing reads; the final
-    //   barrier orders it before the caller reuses the LDS), and a scheduling
-    //   fence that keeps a step's loads ahead of its fragment reads and MFMAs
-    //   (left alone the scheduler issues them after the MFMAs, their registers
-    //   doubling as fragment registers).  A guarded step or store would give
-    //   the loop header a predecessor with the other register set's loads
-    //   outstanding, and the compiler then waits for every load in flight --
-    //   the prefetch one step old included -- before each round's first
-    //   fragment read.
-    // * WK = 1: the guarded form, whose interleaving measured 1-4 % faster on
-    //   these tiles despite that wait; the fence, or a fence before the store
-    //   as well, cost up to 10 %.
-    auto step = [&](int st, auto &lac, auto &lbc, auto &lan, auto &lbn) {
-        lac.load(A, lda, i0, Mo, stage_r(st + T::NR), rend, tid);
-        reprep(lac, st + 2 * T::NR);
-        lbc.load(B, ldb, j0, No, stage_r(st + T::NR), rend, tid, B2);
-        if constexpr (T::WK > 1 && T::SCH == 0) __builtin_amdgcn_sched_barrier(0);
-        float *cur = smem + (st & 1) * (SA + SB);
-        compute(cur, cur + SA);
-        if (T::WK > 1 || T::SCH > 0 || st + 1 < nsteps) {
-            float *nxt = smem + ((st + 1) & 1) * (SA + SB);
-            lan.store(nxt, tid);
-            lbn.store(nxt + SA, tid);
-        }
-        sched_step<T>();
-        __syncthreads();
-    };
-    if constexpr (T::WK > 1 || T::SCH > 0) {
-        int st = 0;
-        if constexpr (T::NR == 2) {
-            for (; st + 1 < nsteps; st += 2) {
-                step(st, la0, lb0, la1, lb1);
-                step(st + 1, la1, lb1, la0, lb0);
-            }
-            if (st < nsteps) step(st, la0, lb0, la1, lb1);
-        } else {
-            for (; st + 2 < nsteps; st += 3) {
-                step(st, la0, lb0, la1, lb1);
-                step(st + 1, la1, lb1, la2, lb2);
-                step(st + 2, la2, lb2, la0, lb0);
-            }
-            if (st < nsteps) step(st, la0, lb0, la1, lb1);
-            if (st + 1 < nsteps) step(st + 1, la1, lb1, la2, lb2);
-        }
-    } else if constexpr (T::NR == 2) {
-        for (int st = 0; st < nsteps; st += 2) {
-            step(st, la0, lb0, la1, lb1);
-            if (st + 1 < nsteps) step(st + 1, la1, lb1, la0, lb0);
-        }
-    } else {
-        for (int st = 0; st < nsteps; st += 3) {
-            step(st, la0, lb0, la1, lb1);
-            if (st + 1 < nsteps) step(st + 1, la1, lb1, la2, lb2);
-            if (st + 2 < nsteps) step(st + 2, la2, lb2, la0, lb0);
-        }
-    }
-}
-
-// put(i, j, v) for every element (i, j) of the tile's valid part (i < Mo,
-// j < No), v its sum.  32x32 MFMA result layout: lane l, register v holds
-// row 8*(v/4) + 4*(l/32) + v%4, column l%32.  With WK > 1 the wave groups'
-// partial tiles go through `red` (LDS, WK*BM*BN floats, free once
-// tile_accumulate has returned) and are summed in wave-group order, so the
-// result does not depend on timing.  STASH: every element's value (valid
-// or not) is also left in red[f], f its fragment-order index (below), for a
-// row-wise epilogue after the next barrier; red must hold TILE floats.
-template <class T, bool STASH = false, class Put>
-__device__ __forceinline__ void tile_epi(const f32x16 (&accs)[T::FM][T::FN][T::NCH], int Mo, int No, int i0,
-                                         int j0, float *__restrict__ red, Put put)
-{
-    const int lane = threadIdx.x & 63;
-    f32x16 acc[T::FM][T::FN];
-#pragma unroll
-    for (int a = 0; a < T::FM; a++)
-#pragma unroll
-        for (int b = 0; b < T::FN; b++) {
-            acc[a][b] = accs[a][b][0];
-#pragma unroll
-            for (int c = 1; c < T::NCH; c++) acc[a][b] += accs[a][b][c];
-        }
-    if constexpr (T::WK == 1) {
-        const int wm = T::wm(), wn = T::wn();
-        const int h = lane >> 5, col = lane & 31;
-        if constexpr (STASH) {
-            const int g = T::wave() % (T::WGM * T::WGN);
-#pragma unroll
-            for (int a = 0; a < T::FM; a++)
-#pragma unroll
-                for (int b = 0; b < T::FN; b++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++)
-                        red[(((g * T::FM + a) * T::FN + b) * 16 + v) * 64 + lane] = acc[a][b][v];
-        }
-#pragma unroll
-        for (int a = 0; a < T::FM; a++)
-#pragma unroll
-            for (int b = 0; b < T::FN; b++) {
-                const int j = j0 + wn * T::WN + b * 32 + col;
-                if (j >= No) continue;
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int i = i0 + wm * T::WM + a * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
-                    if (i < Mo) put(i, j, acc[a][b][v]);
-                }
-            }
-    } else {
-        // fragment-order index of (wave-in-group g, a, b, v, lane)
-        const int g = T::wave() % (T::WGM * T::WGN);
-        float *mine = red + T::wk() * T::TILE;
-#pragma unroll
-        for (int a = 0; a < T::FM; a++)
-#pragma unroll
-            for (int b = 0; b < T::FN; b++)
-#pragma unroll
-                for (int v = 0; v < 16; v++)
-                    mine[(((g * T::FM + a) * T::FN + b) * 16 + v) * 64 + lane] = acc[a][b][v];
-        __syncthreads();
-#pragma unroll 4
-        for (int f = threadIdx.x; f < T::TILE; f += T::THREADS) {
-            float s = red[f];
-#pragma unroll
-            for (int k = 1; k < T::WK; k++) s += red[k * T::TILE + f];
-            const int l = f & 63, v = (f >> 6) & 15, ab = f >> 10;
-            const int b = ab % T::FN, a = (ab / T::FN) % T::FM, gg = ab / (T::FN * T::FM);
-            const int i = i0 + (gg / T::WGN) * T::WM + a * 32 + 8 * (v >> 2) + 4 * (l >> 5) + (v & 3);
-            const int j = j0 + (gg % T::WGN) * T::WN + b * 32 + (l & 31);
-            if (i < Mo && j < No) put(i, j, s);
-            if constexpr (STASH) red[f] = s;     // only this thread reads slot f of slice 0
-        }
-        __syncthreads();            // `red` aliases the stage buffers of the next tile
-    }
-}
-
-// One output element of a tile: a streaming store for the Sched<T, 4 + ..>
-// shapes (it goes past the L2, so the kernel's end does not wait to write
-// back lines the next launch reads through another XCD's L2 anyway).
-template <class T>
-__device__ __forceinline__ void st_out(float *p, float v)
-{
-    if constexpr ((T::SCH & 4) != 0) __builtin_nontemporal_store(v, p);
-    else *p = v;
-}
-
-// C (beta ? += : =) acc for the valid part of the tile.
-template <class T>
-__device__ __forceinline__ void tile_store(const f32x16 (&accs)[T::FM][T::FN][T::NCH], float *__restrict__ C,
-                                           int ldc, int beta, int Mo, int No, int i0, int j0,
-                                           float *__restrict__ red)
-{
-    tile_epi<T>(accs, Mo, No, i0, j0, red, [&](int i, int j, float v) {
-        float *p = C + (size_t)i * ldc + j;
-        st_out<T>(p, beta ? (*p + v) : v);
-    });
-}
-
-// C = acc (beta 0) and, for every 32-column block of each valid row, the dot
-// product of the block with the same block of O:  out[i][j / 32] =
-// sum_{c < 32} C[i][32 (j / 32) + c] O[i][32 (j / 32) + c] (O with C's row
-// stride, out [Mo][No / 32]).  This is the attention backward's per-row term
-// D = dO . O of each 32-wide head (tinylm.c:750-768) formed where dO is made
-// (the O-projection backward's dX tile), in the dQ item's order: two 16-term
-// fma chains, then their sum.  Needs No % 32 == 0 and TILE <= the LDS the
-// tile's stages use (every shape but the 128 x 128 ones; the host checks).
-template <class T>
-__device__ __forceinline__ void tile_store_dot(const f32x16 (&accs)[T::FM][T::FN][T::NCH], float *__restrict__ C,
-                                               int ldc, int Mo, int No, int i0, int j0, const float *__restrict__ O,
-                                               float *__restrict__ out, float *__restrict__ red)
-{
-    if constexpr (T::TILE <= T::lds_max()) {
-        tile_epi<T, true>(accs, Mo, No, i0, j0, red,
-                          [&](int i, int j, float v) { st_out<T>(C + (size_t)i * ldc + j, v); });
-        __syncthreads();
-        // eight lanes per (row, block), lane q holding float4 q of the block
-        // (a wave's O loads: eight 128-byte row segments); each half's chain
-        // passes through its four lanes in order, lane q continuing the sum
-        // lane q - 1 ended with.  Every count here is a multiple of 64, so
-        // whole waves take part in the shuffles.
-        constexpr int NB = T::BN / 32;
-        static_assert(T::BM * NB * 8 % 64 == 0, "whole waves");
-        const int q = threadIdx.x & 7;
-        for (int p8 = threadIdx.x; p8 < T::BM * NB * 8; p8 += T::THREADS) {
-            const int p = p8 >> 3, row = p / NB, cb = p % NB;
-            const int i = i0 + row, jb = j0 + cb * 32;
-            // fragment-order index of (row, column 0 of block cb)
-            const int rr = row % T::WM, a = rr / 32, r32 = rr % 32;
-            const int v = 4 * (r32 >> 3) + (r32 & 3), hb = (r32 >> 2) & 1;
-            const int b = ((cb * 32) % T::WN) / 32;
-            const int g = (row / T::WM) * T::WGN + (cb * 32) / T::WN;
-            const f32x4 x = *reinterpret_cast<const f32x4 *>(
-                red + ((((g * T::FM + a) * T::FN + b) * 16 + v) * 64 + hb * 32) + 4 * q);
-            const int ic = min(i, Mo - 1), jc = min(jb, No - 32);
-            const f32x4 y = *reinterpret_cast<const f32x4 *>(O + (size_t)ic * ldc + jc + 4 * q);
-            float d = 0.f;
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const float in = __shfl_up(d, 1, 4);
-                if ((q & 3) == s) {
-                    float c = s ? in : 0.f;
-                    c += x[0] * y[0];
-                    c += x[1] * y[1];
-                    c += x[2] * y[2];
-                    c += x[3] * y[3];
-                    d = c;
-                }
-            }
-            const float h0 = __shfl_up(d, 4, 8);
-            if (q == 7 && i < Mo && jb < No) out[(size_t)i * (No / 32) + jb / 32] = h0 + d;
-        }
-        __syncthreads();
-    }
-}
-
-// 1 / (1 + e^-z) with the hardware exp2 and reciprocal (within a few ulp of
-// the reference's expf and division; e^-z = inf gives 0, as there).
-__device__ __forceinline__ float hw_sigmoid(float z)
-{
-    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.44269504088896341f));
-}
-
-// LDS of an expert-launch workgroup: the tile's stages or partials, and the
-// SwiGLU epilogue's staged tile beside the partials.
-template <class T>
-__host__ __device__ constexpr int expert_lds()
-{
-    return T::mx(T::lds_max(), (T::WK > 1 ? T::WK * T::TILE : 0) + T::BM * (T::BN + 1));
-}
-
-// SwiGLU epilogue of a paired-column tile (TileLoader PB): tile columns
-// [0, BN/2) hold g = X W1 and [BN/2, BN) hold u = X W3 for the output
-// columns jh + [0, BN/2).  The summed tile goes through LDS (after the WK
-// partials, which it must not overlap) so one thread sees both halves; then
-// a = silu(g) u  (tinylm.c:786, :882) for i < Mo, j < No, and g, u too where
-// Cg / Cu are given.
-template <class T>
-__device__ __forceinline__ void tile_swiglu(const f32x16 (&accs)[T::FM][T::FN][T::NCH], float *__restrict__ Ca,
-                                            float *__restrict__ Cg, float *__restrict__ Cu, int ldc, int Mo,
-                                            int No, int i0, int jh, float *__restrict__ red)
-{
-    constexpr int H = T::BN / 2, LD = T::BN + 1;
-    constexpr int OFF = T::WK > 1 ? T::WK * T::TILE : 0;
-    static_assert(OFF + T::BM * LD <= expert_lds<T>(), "paired tile fits beside the partials");
-    float *L = red + OFF;
-    tile_epi<T>(accs, T::BM, T::BN, 0, 0, red, [&](int i, int j, float v) { L[i * LD + j] = v; });
-    __syncthreads();
-    for (int f = threadIdx.x; f < T::BM * H; f += T::THREADS) {
-        const int x = f / H, c = f % H;
-        const int i = i0 + x, j = jh + c;
-        if (i >= Mo || j >= No) continue;
-        const float g = L[x * LD + c], u = L[x * LD + c + H];
-        const size_t o = (size_t)i * ldc + j;
-        st_out<T>(Ca + o, g * hw_sigmoid(g) * u);
-        if (Cg) st_out<T>(Cg + o, g);
-        if (Cu) st_out<T>(Cu + o, u);
-    }
-    __syncthreads();
-}
-
-template <int FM, int FN, int NCH>
-__device__ __forceinline__ void zero_acc(f32x16 (&acc)[FM][FN][NCH])
-{
-#pragma unroll
-    for (int a = 0; a < FM; a++)
-#pragma unroll
-        for (int b = 0; b < FN; b++)
-#pragma unroll
-            for (int c = 0; c < NCH; c++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) acc[a][b][c][v] = 0.f;
-}
-
-// ------------------------------------------------------- single problem --
-struct GemmArgs {
-    const float *A;
-    const float *B;
-    float *C;
-    int Mo, No, R;
-    int lda, ldb, ldc;
-    int beta;
-    int tiles_n;     // tiles along No
-    int tiles;       // tiles_m * tiles_n
-    int splits;      // workgroups per tile along r
-    int rps;         // r per split (multiple of BK)
-    float *ws;       // splits x Mo x No partials (splits > 1)
-};
-
-template <class T, int LA, int LB, bool VEC>
-__global__ __launch_bounds__(T::THREADS) void k_gemm(GemmArgs g)
-{
-    __shared__ __attribute__((aligned(16))) float smem[T::template lds<LA, LB>()];
-    const int item = xcd_remap(blockIdx.x, gridDim.x);
-    const int z = item / g.tiles, tile = item % g.tiles;
-    const int i0 = (tile / g.tiles_n) * T::BM, j0 = (tile % g.tiles_n) * T::BN;
-    const int rbeg = z * g.rps;
-    const int rend = min(g.R, rbeg + g.rps);
-    f32x16 acc[T::FM][T::FN][T::NCH];
-    zero_acc(acc);
-    tile_accumulate<T, LA, LB, VEC>(smem, g.A, g.B, g.lda, g.ldb, i0, j0, g.Mo, g.No, rbeg, rend, acc);
-    // a split writes its partial (beta 0) into workspace slice z
-    if (g.splits > 1)
-        tile_store<T>(acc, g.ws + (size_t)z * g.Mo * g.No, g.No, 0, g.Mo, g.No, i0, j0, smem);
-    else
-        tile_store<T>(acc, g.C, g.ldc, g.beta, g.Mo, g.No, i0, j0, smem);
-}
-
-// C (beta ? += : =) sum_{z < splits} ws[z], in z order; Mo x No elements.
-__device__ __forceinline__ void reduce_range(const float *__restrict__ ws, float *__restrict__ C,
-                                             int No, int ldc, int splits, int beta,
-                                             size_t e0, size_t e1, size_t n)
-{
-    for (size_t e = e0 + threadIdx.x; e < e1; e += blockDim.x) {
-        float s = ws[e];
-        for (int z = 1; z < splits; z++) s += ws[(size_t)z * n + e];
-        const size_t i = e / (size_t)No, j = e % (size_t)No;
-        float *p = C + i * (size_t)ldc + j;
-        *p = beta ? (*p + s) : s;
-    }
-}
 
 __global__ void k_split_reduce(const float *__restrict__ ws, float *__restrict__ C, int Mo, int No,
                                int ldc, int splits, int beta)
@@ -653,392 +13,6 @@ __global__ void k_split_reduce(const float *__restrict__ ws, float *__restrict__
     const size_t per = 256;
     for (size_t e0 = (size_t)blockIdx.x * per; e0 < n; e0 += (size_t)gridDim.x * per)
         reduce_range(ws, C, No, ldc, splits, beta, e0, e0 + per < n ? e0 + per : n, n);
-}
-
-// ------------------------------------------------------ grouped problems --
-enum { PK_NN = 0, PK_NT = 1, PK_TN = 2, PK_RED = 3, PK_ZERO = 4, PK_COLSUM = 5 };
-#define TLG_ZERO_CHUNK 4096          // floats a clear's work item sets to 0
-#define TLG_MAXSEG 3
-#define TLG_MAXPROB 16                // group_item pins 16 counts
-#define TLG_RED_CHUNK 256
-#define TLG_ERED_CHUNK 2048            // elements per work item of an expert reduction
-
-struct Seg { const float *A, *B; int R, lda, ldb; };
-// The fields every work item reads lie in the first 160 bytes (C to items,
-// then the segments), so a workgroup fetches them in a few scalar loads
-// issued together.
-struct Prob {
-    float *C;
-    const float *ws;      // PK_RED: partials; split GEMM: its partial slice base
-    int Mo, No, ldc, beta;
-    int kind, nseg;
-    int tiles_n, tiles, splits, rps;
-    int items;            // work items: tiles * splits, or reduction chunks
-    Seg seg[TLG_MAXSEG];
-    // Expert-batched problem (nexp > 0): the rows of a top-1 MoE layer are
-    // grouped by expert, expert e owning rows [eoff[e], eoff[e+1]) of every
-    // row operand.  NN / NT: the output rows are expert rows and the weight
-    // operand B of expert e is B + e*es.  TN: the reduction runs over expert
-    // rows in slices of rps, and the output of expert e is C + e*es.  `unit`
-    // is the row extent of one item (BM for NN / NT, rps for TN).
-    const int *eoff;
-    long long es;
-    int nexp, unit;
-    // Fused forms of the MoE expert GEMMs (tinylm.c:876-888, :911-927):
-    //   amap  A rows gathered through it (the sorted row -> token index)
-    //   B2    NN: second weight of a column pair (W3 beside W1), SwiGLU
-    //         epilogue; tiles_n then counts BN/2-column tiles
-    //   epi   TLG_EPI_*: plain store, SwiGLU (C = a, X1 = g, X2 = u when
-    //         given), SwiGLU backward (da from the tile, g / u in X1 / X2
-    //         replaced by dg / du; C unused), or the top-1 combine (C = out,
-    //         out[omap[i]] = fin[..] + gate[..] * tile row i; X1 = the rows
-    //         themselves, sorted order, when given); on a dense NT problem
-    //         ROWDOT: C stored, and X1 [Mo][No/32] the dot of each row's
-    //         32-column blocks with those of `fin` (tile_store_dot)
-    const int *amap, *omap;
-    const float *B2;
-    float *X1, *X2;
-    const float *fin, *gate;
-    int epi;
-};
-// items / devcount: filled from p[] by group_seal() before every launch (0
-// past nprob), so the search for a workgroup's problem reads one contiguous
-// block of counts instead of one problem struct after another.
-struct GroupArgs {
-    int nprob;
-    int rows1;            // expert launches: > 0 = one expert owning rows [0, rows1)
-    int items[TLG_MAXPROB];
-    unsigned devcount;    // bit p: problem p's count is known only on the device (experts)
-    Prob p[TLG_MAXPROB];
-};
-
-// Real work items of an expert-batched problem, from the device-resident
-// row offsets: sum over experts of ceil(rows_e / unit) row units, times the
-// column tiles (NN / NT) or the output tiles (TN).
-__device__ __forceinline__ int expert_items(const Prob &P, const int *eo)
-{
-    int units = 0;
-    for (int e = 0; e < P.nexp; e++) {
-        const int c = eo[e + 1] - eo[e];
-        units += c > 0 ? (c + P.unit - 1) / P.unit : 0;
-    }
-    return units * (P.kind == PK_TN ? P.tiles : P.tiles_n);
-}
-
-// Item -> (expert e, row unit t of that expert, first partial slot of e).
-// Returns false when the item is past the experts' real work.
-__device__ __forceinline__ bool expert_of(const Prob &P, const int *eo, int t, int *e_out, int *t_out,
-                                          int *base, int *rows, int *slot0)
-{
-    int slot = 0;
-    for (int e = 0; e < P.nexp; e++) {
-        const int b = eo[e], c = eo[e + 1] - b;
-        const int n = c > 0 ? (c + P.unit - 1) / P.unit : 0;
-        if (t < n) { *e_out = e; *t_out = t; *base = b; *rows = c; *slot0 = slot; return true; }
-        t -= n;
-        slot += n;
-    }
-    return false;
-}
-
-// Accumulation of one expert tile, with its gather / pair form chosen at run
-// time (uniform per problem): PB only for NN problems.
-template <class T, int LA, int LB>
-__device__ __forceinline__ void expert_acc(float *smem, const Prob &P, const Seg &s, const float *A,
-                                           const float *B, const int *amap, int i0, int j0, int Mo, int No,
-                                           int rbeg, int rend, f32x16 (&acc)[T::FM][T::FN][T::NCH])
-{
-    if constexpr (LA == RC && LB == OC) {
-        if (P.B2) {
-            const float *B2 = P.B2 + (B - s.B);
-            if (amap)
-                tile_accumulate<T, LA, LB, true, true, true>(smem, A, B, s.lda, s.ldb, i0, j0, Mo, No, rbeg,
-                                                             rend, acc, amap, B2);
-            else
-                tile_accumulate<T, LA, LB, true, false, true>(smem, A, B, s.lda, s.ldb, i0, j0, Mo, No, rbeg,
-                                                              rend, acc, nullptr, B2);
-            return;
-        }
-    }
-    if (amap)
-        tile_accumulate<T, LA, LB, true, true>(smem, A, B, s.lda, s.ldb, i0, j0, Mo, No, rbeg, rend, acc, amap);
-    else
-        tile_accumulate<T, LA, LB, true>(smem, A, B, s.lda, s.ldb, i0, j0, Mo, No, rbeg, rend, acc);
-}
-
-template <class T, int LA, int LB>
-__device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int local, const int *eo)
-{
-    f32x16 acc[T::FM][T::FN][T::NCH];
-    int e, t, base, rows, slot0;
-    if (P.kind != PK_TN) {
-        if (!expert_of(P, eo, local / P.tiles_n, &e, &t, &base, &rows, &slot0)) return;
-        // a paired tile covers BN/2 output columns
-        const int i0 = t * T::BM, j0 = (local % P.tiles_n) * (P.B2 ? T::BN / 2 : T::BN);
-        // combine: the tile rows' tokens and gates, staged before the
-        // accumulation so the epilogue waits on one load level, not three
-        __shared__ int s_tok[(LA == RC && LB == OC) ? T::BM : 1];
-        __shared__ float s_gate[(LA == RC && LB == OC) ? T::BM : 1];
-        if constexpr (LA == RC && LB == OC) {
-            if (P.epi == TLG_EPI_COMBINE && (int)threadIdx.x < T::BM) {
-                const int x = threadIdx.x, n = P.omap[base + min(i0 + x, rows - 1)];
-                s_tok[x] = n;
-                s_gate[x] = P.gate[n];
-            }
-        }
-        zero_acc(acc);
-        for (int k = 0; k < P.nseg; k++) {
-            const Seg &s = P.seg[k];
-            // gathered: rows of A through amap[base + x]; else A's expert rows
-            const float *A = P.amap ? s.A : s.A + (size_t)base * s.lda;
-            const int *amap = P.amap ? P.amap + base : nullptr;
-            expert_acc<T, LA, LB>(smem, P, s, A, s.B + (size_t)e * P.es, amap, i0, j0, rows, P.No, 0, s.R,
-                                  acc);
-        }
-        const size_t cb = (size_t)base * P.ldc;
-        switch (P.epi) {
-        case TLG_EPI_SWIGLU:
-            tile_swiglu<T>(acc, P.C + cb, P.X1 ? P.X1 + cb : nullptr, P.X2 ? P.X2 + cb : nullptr, P.ldc, rows,
-                           P.No, i0, j0, smem);
-            break;
-        case TLG_EPI_SWIGLU_BWD: {
-            // In place: g <- da u silu'(g), u <- da silu(g)  (tinylm.c:923-925)
-            float *G = P.X1 + cb, *U = P.X2 + cb;
-            const int ld = P.ldc;
-            tile_epi<T>(acc, rows, P.No, i0, j0, smem, [&](int i, int j, float d) {
-                const size_t o = (size_t)i * ld + j;
-                const float z = G[o], uv = U[o];
-                const float sg = hw_sigmoid(z);
-                const float si = z * sg;
-                const float ds = sg + z * sg * (1.0f - sg);
-                st_out<T>(G + o, d * uv * ds);
-                st_out<T>(U + o, d * si);
-            });
-            break;
-        }
-        case TLG_EPI_COMBINE: {
-            // out[n] = fin[n] + gate[n] y  for token n of sorted row i (:870, :886-888)
-            if constexpr (LA == RC && LB == OC) {
-                __syncthreads();          // the staged tokens, also when the reduction was empty
-                const int ld = P.ldc;
-                float *C = P.C;
-                const float *fin = P.fin;
-                float *Y = P.X1 ? P.X1 + cb : nullptr;      // the expert rows too, when kept
-                tile_epi<T>(acc, rows, P.No, i0, j0, smem, [&](int i, int j, float y) {
-                    const int x = i - i0;
-                    const size_t o = (size_t)s_tok[x] * ld + j;
-                    st_out<T>(C + o, fmaf(s_gate[x], y, fin[o]));
-                    if (Y) st_out<T>(Y + (size_t)i * ld + j, y);
-                });
-            }
-            break;
-        }
-        default:
-            tile_store<T>(acc, P.C + cb, P.ldc, P.beta, rows, P.No, i0, j0, smem);
-        }
-    } else {
-        if (!expert_of(P, eo, local / P.tiles, &e, &t, &base, &rows, &slot0)) return;
-        const int tile = local % P.tiles;
-        const int i0 = (tile / P.tiles_n) * T::BM, j0 = (tile % P.tiles_n) * T::BN;
-        const int rbeg = base + t * P.unit, rend = min(base + rows, rbeg + P.unit);
-        const Seg &s = P.seg[0];
-        zero_acc(acc);
-        // A's reduction rows are sorted rows; gathered ones map through amap
-        expert_acc<T, LA, LB>(smem, P, s, s.A, s.B, P.amap, i0, j0, P.Mo, P.No, rbeg, rend, acc);
-        tile_store<T>(acc, (float *)P.ws + (size_t)(slot0 + t) * P.Mo * P.No, P.No, 0, P.Mo, P.No, i0, j0,
-                      smem);
-    }
-}
-
-// Reduction of an expert TN problem: C_e (beta ? += : =) the sum of expert
-// e's partial slots, in slot order.
-__device__ __forceinline__ void expert_reduce(const Prob &P, int local, const int *eo)
-{
-    const size_t n = (size_t)P.Mo * P.No;
-    const int chunks = (int)((n + TLG_ERED_CHUNK - 1) / TLG_ERED_CHUNK);
-    const int e = local / chunks;
-    int slot0 = 0;
-    for (int k = 0; k < e; k++) {
-        const int c = eo[k + 1] - eo[k];
-        slot0 += c > 0 ? (c + P.unit - 1) / P.unit : 0;
-    }
-    const int c = eo[e + 1] - eo[e];
-    const int ns = c > 0 ? (c + P.unit - 1) / P.unit : 0;
-    const size_t e0 = (size_t)(local % chunks) * TLG_ERED_CHUNK;
-    const size_t e1 = e0 + TLG_ERED_CHUNK < n ? e0 + TLG_ERED_CHUNK : n;
-    float *C = P.C + (size_t)e * P.es;
-    if (ns == 0) {
-        if (!P.beta)
-            for (size_t i = e0 + threadIdx.x; i < e1; i += blockDim.x) C[i] = 0.f;
-        return;
-    }
-    reduce_range(P.ws + (size_t)slot0 * n, C, P.No, P.No, ns, P.beta, e0, e1, n);
-}
-
-template <class T, int LA, int LB, bool EXP>
-__device__ __forceinline__ void group_tile(float *smem, const Prob &P, int local, const int *eo)
-{
-    if constexpr (EXP) {
-        if (P.nexp) { expert_tile<T, LA, LB>(smem, P, local, eo); return; }
-    }
-    const int z = local / P.tiles, tile = local % P.tiles;
-    const int i0 = (tile / P.tiles_n) * T::BM, j0 = (tile % P.tiles_n) * T::BN;
-    f32x16 acc[T::FM][T::FN][T::NCH];
-    zero_acc(acc);
-    if (P.splits > 1) {
-        const Seg &s = P.seg[0];
-        const int rbeg = z * P.rps, rend = min(s.R, rbeg + P.rps);
-        tile_accumulate<T, LA, LB, true>(smem, s.A, s.B, s.lda, s.ldb, i0, j0, P.Mo, P.No, rbeg, rend, acc);
-        tile_store<T>(acc, (float *)P.ws + (size_t)z * P.Mo * P.No, P.No, 0, P.Mo, P.No, i0, j0, smem);
-        return;
-    }
-    for (int k = 0; k < P.nseg; k++) {
-        const Seg &s = P.seg[k];
-        tile_accumulate<T, LA, LB, true>(smem, s.A, s.B, s.lda, s.ldb, i0, j0, P.Mo, P.No, 0, s.R, acc);
-    }
-    if (LA == RC && LB == OC && P.fin) {
-        // mm with its residual add: C = R + acc (R in `fin`, C's layout)
-        float *C = P.C;
-        const float *Rr = P.fin;
-        const int ld = P.ldc;
-        tile_epi<T>(acc, P.Mo, P.No, i0, j0, smem, [&](int i, int j, float v) {
-            const size_t o = (size_t)i * ld + j;
-            st_out<T>(C + o, Rr[o] + v);
-        });
-        return;
-    }
-    if constexpr (LA == RC && LB == RC) {
-        if (P.epi == TLG_EPI_ROWDOT) {
-            tile_store_dot<T>(acc, P.C, P.ldc, P.Mo, P.No, i0, j0, P.fin, P.X1, smem);
-            return;
-        }
-    }
-    tile_store<T>(acc, P.C, P.ldc, P.beta, P.Mo, P.No, i0, j0, smem);
-}
-
-// Work-item mapping of a grouped launch.  The dispatcher deals workgroup b
-// to XCD b % 8; XCD x takes an equal contiguous slice of EVERY problem's
-// items (so each XCD's L2 sees neighbouring tiles of a problem, and every
-// XCD gets the same mix of long and short items), problem by problem in
-// list order (the host lists problems longest item first).  Workgroups past
-// their XCD's share exit at once.
-static_assert(TLG_MAXPROB == 16, "group_item pins exactly 16 item counts");
-__device__ __forceinline__ int group_item(const GroupArgs &g, int b, int *local, const int *eo)
-{
-    const int x = b & 7;
-    int slot = b >> 3;
-    int cnt[TLG_MAXPROB];
-#pragma unroll
-    for (int p = 0; p < TLG_MAXPROB; p++) cnt[p] = g.items[p];
-    const unsigned dev = g.devcount;
-    // every count in flight at once: one round trip, then scalar arithmetic
-    // (counts past nprob are 0, so nprob itself is not needed)
-    asm volatile("" ::"s"(dev), "s"(cnt[0]), "s"(cnt[1]), "s"(cnt[2]), "s"(cnt[3]), "s"(cnt[4]), "s"(cnt[5]),
-                 "s"(cnt[6]), "s"(cnt[7]), "s"(cnt[8]), "s"(cnt[9]), "s"(cnt[10]), "s"(cnt[11]), "s"(cnt[12]),
-                 "s"(cnt[13]), "s"(cnt[14]), "s"(cnt[15]));
-#pragma unroll
-    for (int p = 0; p < TLG_MAXPROB; p++) {
-        // expert-batched GEMMs: the real item count, known only on the device
-        const int n = (dev >> p & 1u) ? expert_items(g.p[p], eo) : cnt[p];
-        const int lo = (x * n) >> 3, hi = ((x + 1) * n) >> 3;
-        if (slot < hi - lo) { *local = lo + slot; return p; }
-        slot -= hi - lo;
-    }
-    return -1;
-}
-
-// `eo`: the expert row offsets of an expert-batched launch, staged in LDS
-// (nullptr for dense launches, which have no expert problems).
-// PK_COLSUM: C[0, No) (beta ? += : =) the sum of the `splits` partial rows
-// ws[z][0, No) (a row-block reduction queued by tlg_defer_colsum).  Item
-// `local` covers float4 columns [4 local, 4 local + 4), one wave per
-// column at a time: lane l adds rows l, l + 64, ... in order, then a fixed
-// butterfly, so the sum does not depend on timing.
-#define TLG_COLSUM_CH 4
-__device__ __forceinline__ void colsum(const Prob &P, int local)
-{
-    const int lane = threadIdx.x & 63, nw = blockDim.x >> 6, w = threadIdx.x >> 6;
-    const int c4 = P.No >> 2, cend = min(TLG_COLSUM_CH * (local + 1), c4);
-    for (int c = TLG_COLSUM_CH * local + w; c < cend; c += nw) {
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
-        for (int z = lane; z < P.splits; z += 64) s += reinterpret_cast<const f32x4 *>(P.ws + (size_t)z * P.No)[c];
-        for (int o = 32; o > 0; o >>= 1) {
-            s.x += __shfl_xor(s.x, o);
-            s.y += __shfl_xor(s.y, o);
-            s.z += __shfl_xor(s.z, o);
-            s.w += __shfl_xor(s.w, o);
-        }
-        if (lane == 0) {
-            f32x4 *out = reinterpret_cast<f32x4 *>(P.C) + c;
-            *out = P.beta ? *out + s : s;
-        }
-    }
-}
-
-template <class T, bool EXP>
-__device__ __forceinline__ void group_body(const GroupArgs &g, float *smem, const int *eo)
-{
-    int local = 0;
-    const int p = group_item(g, blockIdx.x, &local, eo);
-    if (p < 0) return;
-    const Prob &P = g.p[p];
-    // The fields a tile reads first, fetched together: one round trip to the
-    // argument block before the tile's first loads, not one per field.
-    asm volatile("" ::"s"(P.kind), "s"(P.nseg), "s"(P.Mo), "s"(P.No), "s"(P.tiles), "s"(P.tiles_n),
-                 "s"(P.splits), "s"(P.rps), "s"(P.seg[0].A), "s"(P.seg[0].B), "s"(P.seg[0].R), "s"(P.seg[0].lda),
-                 "s"(P.seg[0].ldb));
-    switch (P.kind) {
-    case PK_NN: group_tile<T, RC, OC, EXP>(smem, P, local, eo); break;
-    case PK_NT: group_tile<T, RC, RC, EXP>(smem, P, local, eo); break;
-    case PK_TN: group_tile<T, OC, OC, EXP>(smem, P, local, eo); break;
-    case PK_COLSUM: colsum(P, local); break;
-    case PK_ZERO: {
-        const size_t n = (size_t)P.Mo * P.No, e0 = (size_t)local * TLG_ZERO_CHUNK;
-        const size_t e1 = e0 + TLG_ZERO_CHUNK < n ? e0 + TLG_ZERO_CHUNK : n;
-        for (size_t e = e0 + threadIdx.x; e < e1; e += blockDim.x) P.C[e] = 0.f;
-        break;
-    }
-    default: {
-        if constexpr (EXP) {
-            if (P.nexp) { expert_reduce(P, local, eo); break; }
-        }
-        const size_t n = (size_t)P.Mo * P.No;
-        const size_t e0 = (size_t)local * TLG_RED_CHUNK;
-        const size_t e1 = e0 + TLG_RED_CHUNK < n ? e0 + TLG_RED_CHUNK : n;
-        reduce_range(P.ws, P.C, P.No, P.ldc, P.splits, P.beta, e0, e1, n);
-    }
-    }
-}
-
-template <class T>
-__global__ __launch_bounds__(T::THREADS) void k_group(GroupArgs g)
-{
-    __shared__ __attribute__((aligned(16))) float smem[T::lds_max()];
-    group_body<T, false>(g, smem, nullptr);
-}
-
-// The same code for the expert-batched launches of the MoE layer, under its
-// own name so profiles separate MoE launches from the dense grouped GEMMs.
-// Every problem of such a launch shares one row-offset array; it is staged in
-// LDS once, so finding a work item's expert costs no dependent global loads.
-// The fused variants (gathered rows, paired columns, epilogues) are separate
-// inlined code paths; left alone the compiler gives their accumulators
-// disjoint AGPRs and the kernel drops to 3 waves per SIMD, so it is held to
-// the dense kernels' 4 (no spills at that bound).
-#define TLG_MAX_EXPERTS 64
-template <class T>
-__global__ __launch_bounds__(T::THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_expert_group(GroupArgs g)
-{
-    __shared__ __attribute__((aligned(16))) float smem[expert_lds<T>()];
-    __shared__ int eo[TLG_MAX_EXPERTS + 1];
-    const int E = g.p[0].nexp;
-    if (g.rows1 > 0) {
-        if (threadIdx.x < 2) eo[threadIdx.x] = threadIdx.x ? g.rows1 : 0;
-    } else {
-        for (int i = threadIdx.x; i <= E; i += blockDim.x) eo[i] = g.p[0].eoff[i];
-    }
-    __syncthreads();
-    group_body<T, true>(g, smem, eo);
 }
 
 __global__ void k_zero(float *__restrict__ p, size_t n)
@@ -1060,161 +34,20 @@ int tlg_zero_launch(float *dst, size_t n, hipStream_t st)
 }
 
 // ---------------------------------------------------------------- launch --
-// Tile shapes: BM x BN output per workgroup, BK reduction steps per stage,
-// WGM x WGN waves over the tile, WK wave groups along the reduction.
-struct TileCfg { int bm, bn, bk, wgm, wk, nw; };   // nw 0 = 4 waves
-static const TileCfg kCfgs[] = {
-    {128, 128, 16, 2, 1},   // 0: wave tile 64x64, 4 accumulator chains
-    {128, 64, 32, 2, 1},    // 1: 64x32
-    {64, 128, 32, 2, 1},    // 2: 32x64
-    {64, 64, 32, 2, 1},     // 3: 32x32, one chain per wave
-    {64, 64, 32, 1, 4},     // 4: 64x64 per wave over a quarter of each stage
-    {64, 64, 64, 1, 4},     // 5: same, 64-step stages
-    {64, 128, 32, 1, 2},    // 6: 64x64 per wave, half of each stage
-    {128, 64, 32, 2, 2},    // 7: 64x64 per wave, half of each stage
-    {64, 64, 64, 2, 1},     // 8: 32x32 per wave, 64-step stages
-    {64, 64, 32, 2, 1},     // 9-12: 64x64 tiles (prefetch / chain variants)
-    {64, 64, 32, 2, 1},
-    {64, 64, 32, 2, 1},
-    {64, 64, 32, 2, 1},
-    {32, 64, 32, 1, 2},     // 13: 32x32 per wave, half of each stage
-    {64, 32, 32, 2, 2},     // 14: 32x32 per wave, half of each stage
-    {32, 32, 32, 1, 4},     // 15: 32x32 per wave, a quarter of each stage
-    {64, 64, 32, 2, 1, 2},  // 16: 2 waves, 32x64 per wave
-    {64, 64, 32, 1, 1, 2},  // 17: 2 waves, 64x32 per wave
-    {64, 64, 16, 2, 1},     // 18: 32x32 per wave, 16-step stages
-    {64, 64, 16, 2, 1},     // 19: same, loads three stages ahead
-    {64, 64, 32, 2, 2, 8},  // 20: 8 waves, 32x32 per wave, half of each stage
-    {64, 32, 64, 2, 2},     // 21: 32x32 per wave, half of each 64-step stage
-    {64, 64, 64, 2, 4, 16}, // 22: 16 waves, 32x32 per wave, a quarter of each 64-step stage
-    {64, 64, 64, 2, 2, 8},  // 23: 8 waves, 32x32 per wave, half of each 64-step stage
-    {64, 64, 32, 2, 1},     // 24-25: 3 with a stage's fragment reads first (Sched 1, 2)
-    {64, 64, 32, 2, 1},
-    {64, 32, 32, 2, 2},     // 26: 14, Sched 1
-    {64, 64, 32, 2, 2, 8},  // 27: 20, Sched 1
-    {64, 64, 64, 2, 4, 16}, // 28: 22, Sched 1
-    {32, 64, 32, 1, 2},     // 29: 13, Sched 1
-    {32, 32, 32, 1, 4},     // 30: 15, Sched 1
-    {128, 128, 16, 2, 1},   // 31: 0, Sched 1
-    {128, 64, 32, 2, 1},    // 32: 1, Sched 1
-    {64, 64, 64, 2, 1},     // 33: 8, Sched 1
-    {64, 64, 32, 2, 1},     // 34: 11 (loads three stages ahead), Sched 1
-    {64, 32, 64, 2, 2},     // 35: 21, Sched 1
-    {64, 64, 64, 2, 2, 8},  // 36: 23, Sched 1
-    {64, 64, 16, 2, 1},     // 37: 18, Sched 1
-    {64, 64, 32, 2, 1},     // 38: 3, Sched 1 + streaming stores
-    {64, 64, 16, 2, 1},     // 39: 18, Sched 1 + streaming stores
-    {64, 32, 32, 2, 2},     // 40: 14, Sched 1 + streaming stores
-    {64, 64, 64, 2, 4, 16}, // 41: 22, Sched 1 + streaming stores
-    {64, 64, 32, 2, 2, 8}, // 42: 20, Sched 1 + streaming stores
-    {32, 64, 32, 1, 2},    // 43: 13, Sched 1 + streaming stores
-    {32, 32, 32, 1, 4},    // 44: 15, Sched 1 + streaming stores
-    {128, 128, 16, 2, 1},  // 45: 0, Sched 1 + streaming stores
-    {128, 64, 32, 2, 1},   // 46: 1, Sched 1 + streaming stores
-    {64, 64, 64, 2, 1},    // 47: 8, Sched 1 + streaming stores
-    {64, 64, 32, 2, 1},    // 48: 11, Sched 1 + streaming stores
-    {64, 32, 64, 2, 2},    // 49: 21, Sched 1 + streaming stores
-    {64, 64, 64, 2, 2, 8}, // 50: 23, Sched 1 + streaming stores
-};
+struct TileCfg { int bm, bn, bk, wgm, wk, nr, nw, sch; };
+#define TLG_ROW(i, bm, bn, bk, wgm, wk, nr, nw, sch) {bm, bn, bk, wgm, wk, nr, nw, sch},
+static const TileCfg kCfgs[] = {TLG_TILES(TLG_ROW)};
+#undef TLG_ROW
 static const int kNumCfgs = (int)(sizeof(kCfgs) / sizeof(kCfgs[0]));
-using T0 = Tile<128, 128, 16, 2, 1>;
-using T1 = Tile<128, 64, 32, 2, 1>;
-using T2 = Tile<64, 128, 32, 2, 1>;
-using T3 = Tile<64, 64, 32, 2, 1>;
-using T4 = Tile<64, 64, 32, 1, 4>;
-using T5 = Tile<64, 64, 64, 1, 4>;
-using T6 = Tile<64, 128, 32, 1, 2>;
-using T7 = Tile<128, 64, 32, 2, 2>;
-using T8 = Tile<64, 64, 64, 2, 1>;
-// grouped-launch variants for sweeps: prefetch depth NR, chains per block
-using T9 = Tile<64, 64, 32, 2, 1, 2, 2>;
-using T10 = Tile<64, 64, 32, 2, 1, 2, 1>;
-using T11 = Tile<64, 64, 32, 2, 1, 3, 1>;
-using T12 = Tile<64, 64, 32, 2, 1, 3, 4>;
-using T13 = Tile<32, 64, 32, 1, 2>;
-using T14 = Tile<64, 32, 32, 2, 2>;
-using T15 = Tile<32, 32, 32, 1, 4>;
-using T16 = Tile<64, 64, 32, 2, 1, 2, 0, 2>;
-using T17 = Tile<64, 64, 32, 1, 1, 2, 0, 2>;
-using T18 = Tile<64, 64, 16, 2, 1, 2, 0, 4>;
-using T19 = Tile<64, 64, 16, 2, 1, 3, 0, 4>;
-using T20 = Tile<64, 64, 32, 2, 2, 2, 0, 8>;
-using T21 = Tile<64, 32, 64, 2, 2, 2, 0, 4>;
-using T22 = Tile<64, 64, 64, 2, 4, 2, 0, 16>;
-using T23 = Tile<64, 64, 64, 2, 2, 2, 0, 8>;
-using T24 = Sched<T3, 1>;
-using T25 = Sched<T3, 2>;
-using T26 = Sched<T14, 1>;
-using T27 = Sched<T20, 1>;
-using T28 = Sched<T22, 1>;
-using T29 = Sched<T13, 1>;
-using T30 = Sched<T15, 1>;
-using T31 = Sched<T0, 1>;
-using T32 = Sched<T1, 1>;
-using T33 = Sched<T8, 1>;
-using T34 = Sched<T11, 1>;
-using T35 = Sched<T21, 1>;
-using T36 = Sched<T23, 1>;
-using T37 = Sched<T18, 1>;
-using T38 = Sched<T3, 5>;
-using T39 = Sched<T18, 5>;
-using T40 = Sched<T14, 5>;
-using T41 = Sched<T22, 5>;
-using T42 = Sched<T20, 5>;
-using T43 = Sched<T13, 5>;
-using T44 = Sched<T15, 5>;
-using T45 = Sched<T0, 5>;
-using T46 = Sched<T1, 5>;
-using T47 = Sched<T8, 5>;
-using T48 = Sched<T11, 5>;
-using T49 = Sched<T21, 5>;
-using T50 = Sched<T23, 5>;
 
-template <class T, int LA, int LB>
-static void launch_t(const GemmArgs &a, int grid, bool vec, hipStream_t st)
+// A tile's type as rocprofv3 prints it.
+static int tile_name(const TileCfg &c, char *buf, int len)
 {
-    if (vec) hipLaunchKernelGGL((k_gemm<T, LA, LB, true>), dim3(grid), dim3(256), 0, st, a);
-    else     hipLaunchKernelGGL((k_gemm<T, LA, LB, false>), dim3(grid), dim3(256), 0, st, a);
-}
-
-// Single-call launches of the automatic plan's shapes (0-3) in the Sched<.., 5>
-// form (a stage's fragment reads before its MFMAs, streaming stores) unless
-// TLG_GEMM_SCHED=0.
-static int g_gemm_sched = -1;
-static bool gemm_sched(void)
-{
-    if (g_gemm_sched < 0) {
-        const char *e = getenv("TLG_GEMM_SCHED");
-        g_gemm_sched = (e && *e) ? (atoi(e) != 0) : 1;
-    }
-    return g_gemm_sched != 0;
-}
-
-template <int LA, int LB>
-static void launch_kind(int ci, const GemmArgs &a, int grid, bool vec, hipStream_t st)
-{
-    if (ci <= 3 && gemm_sched()) {
-        switch (ci) {
-        case 0: launch_t<Sched<T0, 5>, LA, LB>(a, grid, vec, st); return;
-        case 1: launch_t<Sched<T1, 5>, LA, LB>(a, grid, vec, st); return;
-        case 2: launch_t<Sched<T2, 5>, LA, LB>(a, grid, vec, st); return;
-        default: launch_t<Sched<T3, 5>, LA, LB>(a, grid, vec, st); return;
-        }
-    }
-    switch (ci) {
-    case 0: launch_t<T0, LA, LB>(a, grid, vec, st); break;
-    case 1: launch_t<T1, LA, LB>(a, grid, vec, st); break;
-    case 2: launch_t<T2, LA, LB>(a, grid, vec, st); break;
-    case 3: launch_t<T3, LA, LB>(a, grid, vec, st); break;
-    case 4: launch_t<T4, LA, LB>(a, grid, vec, st); break;
-    case 5: launch_t<T5, LA, LB>(a, grid, vec, st); break;
-    case 6: launch_t<T6, LA, LB>(a, grid, vec, st); break;
-    case 7: launch_t<T7, LA, LB>(a, grid, vec, st); break;
-    case 13: launch_t<T13, LA, LB>(a, grid, vec, st); break;
-    case 14: launch_t<T14, LA, LB>(a, grid, vec, st); break;
-    case 15: launch_t<T15, LA, LB>(a, grid, vec, st); break;
-    default: launch_t<T8, LA, LB>(a, grid, vec, st); break;
-    }
+    if (c.sch)
+        return snprintf(buf, (size_t)len, "Sched<Tile<%d, %d, %d, %d, %d, %d, %d>, %d>", c.bm, c.bn, c.bk, c.wgm,
+                        c.wk, c.nr, c.nw, c.sch);
+    return snprintf(buf, (size_t)len, "Tile<%d, %d, %d, %d, %d, %d, %d>", c.bm, c.bn, c.bk, c.wgm, c.wk, c.nr,
+                    c.nw);
 }
 
 static inline bool al16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
@@ -1244,25 +77,32 @@ static GemmPlan make_plan(int ci, int Mo, int No, int R, int splits, size_t ws_f
     return p;
 }
 
-// Automatic choice: the largest tile that still yields about one wave of
-// workgroups over the 256 CUs; when even 64x64 tiles are too few (small
-// outputs with long reductions, i.e. mm_atb's dW), split the reduction so
-// every split keeps >= 256 reduction steps.
+// Automatic choice: the largest of 128x128, 64x64 and 32x32 tiles that gives
+// the 256 CUs about 160 work items, splitting the reduction as far as every
+// split keeps >= 512 steps (small outputs with long reductions, i.e. mm_atb's
+// dW).  Measured, best other shape against the rule's: mm (8192, 384, 2048)
+// 128x128 79 us, 128x64 83, 64x64 103; mm (4096, 768, 256) 64x64 14.5,
+// 32x32 20.2; mm (2048, 512, 128) 32x32 7.3, 64x64 10.7; mm_atb
+// (8192, 1024, 384) 8 splits of 128x128 47.5, 64x64 51.4.  64x64 tiles take
+// 64-step stages (8 waves, a quarter of each stage per wave) from 512 steps
+// on and 16-step stages below: 14.5 against 16.8 us at 768 steps, 7.5 against
+// 8.0 at 128.
 static GemmPlan plan_gemm(int Mo, int No, int R, size_t ws_floats)
 {
     if (g_force_cfg >= 0 && g_force_cfg < kNumCfgs)
         return make_plan(g_force_cfg, Mo, No, R, g_force_splits, ws_floats);
-    static const int order[] = {0, 1, 2, 3};
-    for (int k = 0; k < 4; k++) {
+    const int enough = 160, maxs = R / 512 > 1 ? R / 512 : 1;
+    const int order[] = {9, R >= 512 ? 8 : 3, 15};
+    int ci = 15, splits = 1;
+    for (int k = 0; k < 3; k++) {
         const TileCfg &c = kCfgs[order[k]];
-        const int tiles = cdiv(Mo, c.bm) * cdiv(No, c.bn);
-        if (tiles >= 240) return make_plan(order[k], Mo, No, R, 1, ws_floats);
+        const long long tiles = (long long)cdiv(Mo, c.bm) * cdiv(No, c.bn);
+        ci = order[k];
+        splits = tiles >= enough ? 1 : cdiv(enough, (int)tiles);
+        if (splits > maxs) splits = maxs;
+        if (tiles * splits >= enough) break;
     }
-    const int tiles = cdiv(Mo, 64) * cdiv(No, 64);
-    int splits = cdiv(256, tiles);
-    const int maxs = R / 256 > 1 ? R / 256 : 1;
-    if (splits > maxs) splits = maxs;
-    return make_plan(3, Mo, No, R, splits, ws_floats);
+    return make_plan(ci, Mo, No, R, splits, ws_floats);
 }
 
 // Name of the kernel instance a device-pointer call with aligned operands
@@ -1285,12 +125,11 @@ int tlg_describe(TlgKind kind, int Mo, int No, int R, char *buf, int len, int *s
     const int la = (kind == TLG_TN) ? OC : RC;
     const int lb = (kind == TLG_NT) ? RC : OC;
     const bool vec = (la == RC ? (R % 4 == 0) : (Mo % 4 == 0)) && (lb == RC ? (R % 4 == 0) : (No % 4 == 0));
-    if (p.ci <= 3 && gemm_sched())
-        snprintf(buf, (size_t)len, "k_gemm<Sched<Tile<%d, %d, %d, %d, %d, 2, 0, 4>, 5>, %d, %d, %s>", c.bm, c.bn,
-                 c.bk, c.wgm, c.wk, la, lb, vec ? "true" : "false");
-    else
-        snprintf(buf, (size_t)len, "k_gemm<Tile<%d, %d, %d, %d, %d, 2, 0, 4>, %d, %d, %s>", c.bm, c.bn, c.bk,
-                 c.wgm, c.wk, la, lb, vec ? "true" : "false");
+    char tile[96];
+    TileCfg t = c;
+    t.sch = 5;                                   // single calls
+    tile_name(t, tile, (int)sizeof tile);
+    snprintf(buf, (size_t)len, "k_gemm<%s, %d, %d, %s>", tile, la, lb, vec ? "true" : "false");
     if (splits) *splits = p.splits;
     return TLG_OK;
 }
@@ -1345,9 +184,8 @@ static int gemm_launch_ws(TlgKind kind, const float *A, const float *B, float *C
     a.splits = pl.splits; a.rps = pl.rps;
     a.ws = ws;
     const int grid = pl.tiles * pl.splits;
-    if (la == RC && lb == OC)      launch_kind<RC, OC>(pl.ci, a, grid, vec, st);
-    else if (la == RC && lb == RC) launch_kind<RC, RC>(pl.ci, a, grid, vec, st);
-    else                           launch_kind<OC, OC>(pl.ci, a, grid, vec, st);
+    if (!tlg_single_part0(pl.ci, kind, vec, a, grid, st) && !tlg_single_part1(pl.ci, kind, vec, a, grid, st))
+        return tlg_fail(TLG_EINVAL, "GEMM: no kernel for tile configuration %d", pl.ci);
     TLG_HIP(hipGetLastError());
     if (pl.splits > 1) return launch_reduce(ws, C, Mo, No, ldc, pl.splits, beta, st);
     return TLG_OK;
@@ -1443,30 +281,34 @@ static int g_ws_half = 0;
 static int flush_foreign(hipStream_t st);
 
 // Tile shape of a grouped launch (all problems of a group share it): the
-// first candidate that still gives every CU `g_min_waves` workgroups, else
-// the last.  Measured on MI355X over the m3 training step (graph replay):
-// 64x64 tiles where a launch has >= 3 x 256 of them, else 64x32 tiles whose
-// two wave pairs split each stage's reduction (more, smaller work items and
-// 5 waves per SIMD instead of 4), with dW splits of about 512 reduction
-// steps: 1.548 ms/step, against 1.637 for 64x64 tiles and 384-step splits
-// (m8: 6.95 against 7.91 ms).  TLG_GROUP_CANDS, TLG_GROUP_MINWAVES and
-// TLG_GROUP_RTARGET (or tlg_tune_group_policy) override the policy,
-// tlg_tune_group pins one shape.
+// first row of kAuto whose shape gives the launch enough work items.  Measured
+// over the nano, m3 and m8 models' launches (replayed, us; the row's shape
+// against the next one's):
+//   128x128  m8 FFN backward 186 / 203 (128x64), m3 60 / 73; m8 W2 48 / 50.
+//            Launches without an mm_atb need whole rounds of 256 items (m8
+//            Q | K | V: 320 items, 35 against 32 on 64x64 tiles); short
+//            reductions run it in the compiler's order with streaming stores
+//            (m3 logits 27 / 30).
+//   128x64   m3 head backward 62 / 67 (64x64)
+//   64x64    m3 Q | K | V 10.5 / 11.3, its backward 21.7 / 22.3
+//   64x64 of 8 waves, each 64x32 of a quarter of a 64-step stage: one item per
+//            CU, so the waves come from the reduction (m3 W2 16.1 / 18.8)
+//   64x32, 32x32 likewise (nano head backward 23 / 28 / 29, W2 7.0 on 32x32)
+// mm_atb splits aim for about 512 reduction steps.  TLG_GROUP_CANDS,
+// TLG_GROUP_MINWAVES and TLG_GROUP_RTARGET (or tlg_tune_group_policy) put a
+// list of their own in its place, tlg_tune_group pins one shape.
+static const struct { int cfg, items; } kAuto[] = {{33, 160}, {34, 240}, {35, 320}, {41, 160}, {21, 128}, {15, 0}};
 static int g_group_cfg = -1;
 static int g_group_rt = 0;               // split target pinned for the next launches (tlg_tune_group_split)
 static double g_min_waves = 3.0;
-static int g_cand[4] = {24, 26, -1, -1};  // 64x64, then 64x32 (2 x 2 waves), both in the Sched<.., 1> order
+static int g_cand[4] = {-1, -1, -1, -1};  // candidates put in place of kAuto
 static int g_rtarget = 512;
 static int g_erps = 1024;                // expert TN slice (TLG_EXPERT_RPS)
 static int g_expert_cfg = -1;            // expert tile shape pinned (TLG_EXPERT_CFG: 3, 14, 15, 18, 22)
-static int g_expert_sched = -1;          // expert tiles: 0 the compiler's order, 1 Sched<.., 1>, 2 Sched<.., 5>
-                                         // (that order with streaming stores), -1 automatic: 2 for launches of
+static int g_expert_sched = -1;          // expert tiles: 0, 1 plain stores, 2 streaming ones, -1 automatic: 2 for launches of
                                          // dense rows (the training step's fused SwiGLU: 2.003 -> 1.995 ms), 1 for
                                          // MoE launches (streaming measured 0.232 -> 0.237 ms per kept pair: the
                                          // next launch reads their g, u, a, y right away) (TLG_EXPERT_SCHED)
-static int g_expert_bk16 = 1;            // 64x64 expert tiles with 16-step stages (TLG_EXPERT_BK16=0: 32-step)
-static int g_expert_w16 = 0;             // 16-wave 64x64 tiles for launches short of 64x64 items (TLG_EXPERT_W16=1;
-                                         // measured slower: kept MoE pair 0.2345 -> 0.2489 ms)
 static int g_group_last = 3;          // shape of the most recent grouped launch
 static const char *g_group_last_name = nullptr;   // set when that launch was a GEMV group
 
@@ -1495,8 +337,6 @@ static void group_env(void)
     if (e && (atoi(e) == 3 || atoi(e) == 14 || atoi(e) == 15 || atoi(e) == 18 || atoi(e) == 22))
         g_expert_cfg = atoi(e);
     if ((e = getenv("TLG_EXPERT_SCHED")) && atoi(e) >= -1 && atoi(e) <= 2) g_expert_sched = atoi(e);
-    if ((e = getenv("TLG_EXPERT_W16"))) g_expert_w16 = atoi(e) != 0;
-    if ((e = getenv("TLG_EXPERT_BK16"))) g_expert_bk16 = atoi(e) != 0;
     e = getenv("TLG_GROUP_RTARGET");
     if (e && atoi(e) >= 64) g_rtarget = atoi(e);
 }
@@ -1514,63 +354,13 @@ static const GroupArgs &group_seal(const GroupArgs &a)
     return b;
 }
 
-template <class T>
-static void lgroup(const GroupArgs &a, int grid, hipStream_t st)
-{
-    hipLaunchKernelGGL((k_group<T>), dim3(grid), dim3(T::THREADS), 0, st, group_seal(a));
-}
-
 static void launch_group(int ci, const GroupArgs &a, int grid, hipStream_t st)
 {
-    switch (ci) {
-    case 0: lgroup<T0>(a, grid, st); break;
-    case 1: lgroup<T1>(a, grid, st); break;
-    case 4: lgroup<T4>(a, grid, st); break;
-    case 8: lgroup<T8>(a, grid, st); break;
-    case 9: lgroup<T9>(a, grid, st); break;
-    case 10: lgroup<T10>(a, grid, st); break;
-    case 11: lgroup<T11>(a, grid, st); break;
-    case 12: lgroup<T12>(a, grid, st); break;
-    case 13: lgroup<T13>(a, grid, st); break;
-    case 14: lgroup<T14>(a, grid, st); break;
-    case 15: lgroup<T15>(a, grid, st); break;
-    case 16: lgroup<T16>(a, grid, st); break;
-    case 17: lgroup<T17>(a, grid, st); break;
-    case 18: lgroup<T18>(a, grid, st); break;
-    case 19: lgroup<T19>(a, grid, st); break;
-    case 20: lgroup<T20>(a, grid, st); break;
-    case 21: lgroup<T21>(a, grid, st); break;
-    case 22: lgroup<T22>(a, grid, st); break;
-    case 23: lgroup<T23>(a, grid, st); break;
-    case 24: lgroup<T24>(a, grid, st); break;
-    case 25: lgroup<T25>(a, grid, st); break;
-    case 26: lgroup<T26>(a, grid, st); break;
-    case 27: lgroup<T27>(a, grid, st); break;
-    case 28: lgroup<T28>(a, grid, st); break;
-    case 29: lgroup<T29>(a, grid, st); break;
-    case 30: lgroup<T30>(a, grid, st); break;
-    case 31: lgroup<T31>(a, grid, st); break;
-    case 32: lgroup<T32>(a, grid, st); break;
-    case 33: lgroup<T33>(a, grid, st); break;
-    case 34: lgroup<T34>(a, grid, st); break;
-    case 35: lgroup<T35>(a, grid, st); break;
-    case 36: lgroup<T36>(a, grid, st); break;
-    case 37: lgroup<T37>(a, grid, st); break;
-    case 38: lgroup<T38>(a, grid, st); break;
-    case 39: lgroup<T39>(a, grid, st); break;
-    case 40: lgroup<T40>(a, grid, st); break;
-    case 41: lgroup<T41>(a, grid, st); break;
-    case 42: lgroup<T42>(a, grid, st); break;
-    case 43: lgroup<T43>(a, grid, st); break;
-    case 44: lgroup<T44>(a, grid, st); break;
-    case 45: lgroup<T45>(a, grid, st); break;
-    case 46: lgroup<T46>(a, grid, st); break;
-    case 47: lgroup<T47>(a, grid, st); break;
-    case 48: lgroup<T48>(a, grid, st); break;
-    case 49: lgroup<T49>(a, grid, st); break;
-    case 50: lgroup<T50>(a, grid, st); break;
-    default: lgroup<T3>(a, grid, st); break;
-    }
+    if (ci < 0 || ci >= kNumCfgs) ci = 3;
+    const GroupArgs &b = group_seal(a);
+#define TLG_TRY(k) if (!tlg_group_part##k(ci, b, grid, st))
+    TLG_TILE_PARTS(TLG_TRY) {}
+#undef TLG_TRY
     g_group_last = ci;
     g_group_last_name = nullptr;
 }
@@ -1581,7 +371,7 @@ extern "C" int tlg_tune_group_policy(const int *cands, int ncands, double min_wa
     if (ncands < 0 || ncands > 3 || (ncands > 0 && !cands) || min_waves < 0 || (rtarget && rtarget < 64))
         return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: bad arguments");
     for (int k = 0; k < ncands; k++)
-        if (cands[k] < 0 || cands[k] >= kNumCfgs || cands[k] == 2 || (cands[k] >= 5 && cands[k] <= 7))
+        if (cands[k] < 0 || cands[k] >= kNumCfgs)
             return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: config %d", cands[k]);
     if (ncands > 0) {
         for (int k = 0; k < ncands; k++) g_cand[k] = cands[k];
@@ -1604,7 +394,7 @@ extern "C" int tlg_tune_expert(int cfg, int sched)
 
 extern "C" int tlg_tune_group(int cfg)
 {
-    if (cfg != -1 && cfg != 0 && cfg != 1 && cfg != 3 && cfg != 4 && (cfg < 8 || cfg >= kNumCfgs))
+    if (cfg < -1 || cfg >= kNumCfgs)
         return tlg_fail(TLG_EINVAL, "tlg_tune_group: config %d", cfg);
     g_group_cfg = cfg;
     return TLG_OK;
@@ -1621,55 +411,11 @@ extern "C" int tlg_tune_group_split(int rtarget)
 const char *tlg_group_kernel_name(void)
 {
     if (g_group_last_name) return g_group_last_name;
-    switch (g_group_last) {
-    case 0: return "k_group<Tile<128, 128, 16, 2, 1, 2, 0, 4> >";
-    case 1: return "k_group<Tile<128, 64, 32, 2, 1, 2, 0, 4> >";
-    case 4: return "k_group<Tile<64, 64, 32, 1, 4, 2, 0, 4> >";
-    case 8: return "k_group<Tile<64, 64, 64, 2, 1, 2, 0, 4> >";
-    case 9: return "k_group<Tile<64, 64, 32, 2, 1, 2, 2, 4> >";
-    case 10: return "k_group<Tile<64, 64, 32, 2, 1, 2, 1, 4> >";
-    case 11: return "k_group<Tile<64, 64, 32, 2, 1, 3, 1, 4> >";
-    case 12: return "k_group<Tile<64, 64, 32, 2, 1, 3, 4, 4> >";
-    case 13: return "k_group<Tile<32, 64, 32, 1, 2, 2, 0, 4> >";
-    case 14: return "k_group<Tile<64, 32, 32, 2, 2, 2, 0, 4> >";
-    case 15: return "k_group<Tile<32, 32, 32, 1, 4, 2, 0, 4> >";
-    case 16: return "k_group<Tile<64, 64, 32, 2, 1, 2, 0, 2> >";
-    case 17: return "k_group<Tile<64, 64, 32, 1, 1, 2, 0, 2> >";
-    case 18: return "k_group<Tile<64, 64, 16, 2, 1, 2, 0, 4> >";
-    case 19: return "k_group<Tile<64, 64, 16, 2, 1, 3, 0, 4> >";
-    case 20: return "k_group<Tile<64, 64, 32, 2, 2, 2, 0, 8> >";
-    case 21: return "k_group<Tile<64, 32, 64, 2, 2, 2, 0, 4> >";
-    case 22: return "k_group<Tile<64, 64, 64, 2, 4, 2, 0, 16> >";
-    case 23: return "k_group<Tile<64, 64, 64, 2, 2, 2, 0, 8> >";
-    case 24: return "k_group<Sched<Tile<64, 64, 32, 2, 1, 2, 0, 4>, 1> >";
-    case 25: return "k_group<Sched<Tile<64, 64, 32, 2, 1, 2, 0, 4>, 2> >";
-    case 26: return "k_group<Sched<Tile<64, 32, 32, 2, 2, 2, 0, 4>, 1> >";
-    case 27: return "k_group<Sched<Tile<64, 64, 32, 2, 2, 2, 0, 8>, 1> >";
-    case 28: return "k_group<Sched<Tile<64, 64, 64, 2, 4, 2, 0, 16>, 1> >";
-    case 29: return "k_group<Sched<Tile<32, 64, 32, 1, 2, 2, 0, 4>, 1> >";
-    case 30: return "k_group<Sched<Tile<32, 32, 32, 1, 4, 2, 0, 4>, 1> >";
-    case 31: return "k_group<Sched<Tile<128, 128, 16, 2, 1, 2, 0, 4>, 1> >";
-    case 32: return "k_group<Sched<Tile<128, 64, 32, 2, 1, 2, 0, 4>, 1> >";
-    case 33: return "k_group<Sched<Tile<64, 64, 64, 2, 1, 2, 0, 4>, 1> >";
-    case 34: return "k_group<Sched<Tile<64, 64, 32, 2, 1, 3, 1, 4>, 1> >";
-    case 35: return "k_group<Sched<Tile<64, 32, 64, 2, 2, 2, 0, 4>, 1> >";
-    case 36: return "k_group<Sched<Tile<64, 64, 64, 2, 2, 2, 0, 8>, 1> >";
-    case 37: return "k_group<Sched<Tile<64, 64, 16, 2, 1, 2, 0, 4>, 1> >";
-    case 38: return "k_group<Sched<Tile<64, 64, 32, 2, 1, 2, 0, 4>, 5> >";
-    case 39: return "k_group<Sched<Tile<64, 64, 16, 2, 1, 2, 0, 4>, 5> >";
-    case 40: return "k_group<Sched<Tile<64, 32, 32, 2, 2, 2, 0, 4>, 5> >";
-    case 41: return "k_group<Sched<Tile<64, 64, 64, 2, 4, 2, 0, 16>, 5> >";
-    case 42: return "k_group<Sched<Tile<64, 64, 32, 2, 2, 2, 0, 8>, 5> >";
-    case 43: return "k_group<Sched<Tile<32, 64, 32, 1, 2, 2, 0, 4>, 5> >";
-    case 44: return "k_group<Sched<Tile<32, 32, 32, 1, 4, 2, 0, 4>, 5> >";
-    case 45: return "k_group<Sched<Tile<128, 128, 16, 2, 1, 2, 0, 4>, 5> >";
-    case 46: return "k_group<Sched<Tile<128, 64, 32, 2, 1, 2, 0, 4>, 5> >";
-    case 47: return "k_group<Sched<Tile<64, 64, 64, 2, 1, 2, 0, 4>, 5> >";
-    case 48: return "k_group<Sched<Tile<64, 64, 32, 2, 1, 3, 1, 4>, 5> >";
-    case 49: return "k_group<Sched<Tile<64, 32, 64, 2, 2, 2, 0, 4>, 5> >";
-    case 50: return "k_group<Sched<Tile<64, 64, 64, 2, 2, 2, 0, 8>, 5> >";
-    default: return "k_group<Tile<64, 64, 32, 2, 1, 2, 0, 4> >";
-    }
+    static char name[128];
+    char tile[96];
+    tile_name(kCfgs[g_group_last], tile, (int)sizeof tile);
+    snprintf(name, sizeof name, "k_group<%s >", tile);
+    return name;
 }
 
 // Grid for the XCD-sliced mapping of group_item: 8 x the largest per-XCD
@@ -1931,25 +677,41 @@ int tlg_group_launch(const TlgGemmCall *calls, int n, hipStream_t st)
     // (or the pinned target)
     const int rtarget = g_group_rt > 0 ? g_group_rt : rmax > g_rtarget ? rmax : g_rtarget;
 
-    // tile shape: pinned, or the largest with >= g_min_waves waves of items
-    int ci = g_group_cfg;
-    if (ci < 0) {
-        int last = 24;
-        ci = -1;
-        for (int k = 0; k < 4 && g_cand[k] >= 0 && ci < 0; k++) {
-            last = g_cand[k];
-            const TileCfg &tc = kCfgs[g_cand[k]];
-            double items = 0;
-            for (int i = 0; i < n; i++) {
-                if (probs[i].kind == PK_ZERO) continue;
-                const double tiles = (double)cdiv(probs[i].Mo, tc.bm) * cdiv(probs[i].No, tc.bn);
-                const double sp = (probs[i].kind == PK_TN && Rtot[i] > rtarget + rtarget / 2)
-                                ? (double)cdiv(Rtot[i], rtarget) : 1.0;
-                items += tiles * sp;
-            }
-            if (items >= g_min_waves * 256) ci = g_cand[k];
+    // tile shape: pinned, or by the work items it gives the launch
+    auto items_of = [&](int cfg) {
+        const TileCfg &tc = kCfgs[cfg];
+        double items = 0;
+        for (int i = 0; i < n; i++) {
+            if (probs[i].kind == PK_ZERO) continue;
+            const double tiles = (double)cdiv(probs[i].Mo, tc.bm) * cdiv(probs[i].No, tc.bn);
+            const double sp = (probs[i].kind == PK_TN && Rtot[i] > rtarget + rtarget / 2)
+                            ? (double)cdiv(Rtot[i], rtarget) : 1.0;
+            items += tiles * sp;
         }
-        if (ci < 0) ci = last;                 // smallest candidate
+        return items;
+    };
+    int ci = g_group_cfg;
+    if (ci < 0 && g_cand[0] >= 0) {
+        for (int k = 0; k < 4 && g_cand[k] >= 0; k++) {
+            ci = g_cand[k];                    // the last one if none is enough
+            if (items_of(ci) >= g_min_waves * 256) break;
+        }
+    } else if (ci < 0) {
+        bool tn = false;
+        for (int i = 0; i < n; i++) tn = tn || probs[i].kind == PK_TN;
+        for (const auto &row : kAuto) {
+            ci = row.cfg;
+            const double items = items_of(ci);
+            if (items < row.items) continue;
+            if (ci == 33 && !tn) {
+                const double rounds = items / 256.0;
+                if (rounds < 2.0 && rounds / (rounds > 1.0 ? 2.0 : 1.0) < 0.7) continue;
+                if (rounds < 1.0 && rmax <= 512) continue;
+                if (rmax <= 512) ci = 47;
+            }
+            if (ci == 34 && !tn) continue;
+            break;
+        }
     }
     // the block-dot epilogue stages a whole tile in the stage buffers: not on
     // the 128 x 128 shapes, whose tile is larger than their stages
@@ -2032,11 +794,16 @@ static int flush_foreign(hipStream_t st)
     return TLG_OK;
 }
 
+// Launches of expert reductions alone
+static void launch_reductions(const GroupArgs &a, hipStream_t st)
+{
+    (void)tlg_expert_part(3, group_seal(a), group_grid(a), st);
+}
+
 static int ecarry_flush(hipStream_t st)
 {
     if (!g_ecarry.nprob) return TLG_OK;
-    hipLaunchKernelGGL((k_expert_group<T3>), dim3(group_grid(g_ecarry)), dim3(T3::THREADS), 0, st,
-                       group_seal(g_ecarry));
+    launch_reductions(g_ecarry, st);
     g_ecarry.nprob = 0;
     g_ecarry_used = 0;
     TLG_HIP(hipGetLastError());
@@ -2054,7 +821,7 @@ static int ecarry_flush_with_pending(hipStream_t st, bool *done)
     if (!g_ecarry.nprob || !g_npending || g_ecarry.nprob + g_npending > TLG_MAXPROB) return TLG_OK;
     GroupArgs a = g_ecarry;
     add_reductions(a);
-    hipLaunchKernelGGL((k_expert_group<T3>), dim3(group_grid(a)), dim3(T3::THREADS), 0, st, group_seal(a));
+    launch_reductions(a, st);
     g_ecarry.nprob = 0;
     g_ecarry_used = 0;
     TLG_HIP(hipGetLastError());
@@ -2098,6 +865,15 @@ int tlg_group_drain(hipStream_t st)
     g_ecarry_eoff = nullptr;
     g_ws_half = 0;
     return rc;
+}
+
+// Extents of an expert shape.
+static TileCfg expert_shape(int key)
+{
+#define TLG_ROW(k, bm, bn, bk, wgm, wk, nw) if (key == k) return TileCfg{bm, bn, bk, wgm, wk, 2, nw, 0};
+    TLG_EXPERTS(TLG_ROW)
+#undef TLG_ROW
+    return expert_shape(15);
 }
 
 int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E, int rows, hipStream_t st,
@@ -2209,11 +985,9 @@ int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E,
     if (need(rps) > g_tlg.ws_floats)
         return tlg_fail(TLG_ENOMEM, "expert launch: %d experts' partials exceed the workspace", E);
 
-    // tile shape: the largest of 64x64, 64x32 (2 x 2 waves) and 32x32 (a
-    // quarter stage per wave) that gives about g_min_waves x 256 items, as
-    // for dense grouped launches (measured at configs[4]: W2's N = 256
-    // launches run 15 % faster on 32x32 tiles than on 64x32; the 8-wave
-    // 64x64 tile was slower on every expert launch)
+    // tile shape: the largest of 64x64, 64x32 and 32x32 that gives about 320
+    // items (the m3 MoE layer 243 us on 64x64 tiles, 267 on 64x32, 246 on
+    // 128x128, whose SwiGLU epilogue costs the m8 step 1 %)
     auto items_for = [&](const TileCfg &c) {
         double t = 0;
         for (int i = 0; i < n; i++) {
@@ -2223,15 +997,10 @@ int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E,
         }
         return t;
     };
-    const double enough = g_min_waves * 256;
-    // (TLG_EXPERT_W16=1: launches with fewer 64x64 items than that but about
-    // one per CU -- the N = 256 W2 launches -- run 64x64 tiles of 16 waves,
-    // as the dense W2 forward does; slower on every configs[4] launch)
     const int ci = g_expert_cfg >= 0 ? g_expert_cfg
-                 : items_for(kCfgs[3]) >= enough ? (g_expert_bk16 ? 18 : 3)
-                 : (g_expert_w16 && items_for(kCfgs[22]) >= 240) ? 22
-                 : items_for(kCfgs[14]) >= enough ? 14 : 15;
-    const TileCfg &tc = kCfgs[ci];
+                 : items_for(expert_shape(3)) >= 320 ? 3
+                 : items_for(expert_shape(14)) >= 320 ? 14 : 15;
+    const TileCfg tc = expert_shape(ci);
     GroupArgs a, red, pend;
     a.nprob = red.nprob = pend.nprob = 0;
     a.rows1 = red.rows1 = pend.rows1 = dense ? rows : 0;
@@ -2286,21 +1055,11 @@ int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E,
     // an XCD's share of the real items can exceed its share of the upper
     // bound by one per expert problem
     static_assert(sizeof(GroupArgs) <= 4096, "kernel arguments");
-    const dim3 eg(group_grid(a) + 8 * n);
-    // +100: the Sched<.., 1> order; +200: that order with streaming stores
-    const int key = ci + 100 * (g_expert_sched >= 0 ? g_expert_sched : dense ? 2 : 1);
-#define TLG_EXPERT_CASE(k, TT)                                                                                  \
-    case k: hipLaunchKernelGGL((k_expert_group<TT>), eg, dim3(TT::THREADS), 0, st, group_seal(a)); break;
-    switch (key) {
-    TLG_EXPERT_CASE(3, T3) TLG_EXPERT_CASE(14, T14) TLG_EXPERT_CASE(15, T15) TLG_EXPERT_CASE(18, T18)
-    TLG_EXPERT_CASE(22, T22)
-    TLG_EXPERT_CASE(103, T24) TLG_EXPERT_CASE(114, T26) TLG_EXPERT_CASE(115, T30) TLG_EXPERT_CASE(118, T37)
-    TLG_EXPERT_CASE(122, T28)
-    TLG_EXPERT_CASE(203, T38) TLG_EXPERT_CASE(214, T40) TLG_EXPERT_CASE(215, T44) TLG_EXPERT_CASE(218, T39)
-    TLG_EXPERT_CASE(222, T41)
-    default: return tlg_fail(TLG_EINVAL, "expert launch: no kernel for tile form %d", key);
-    }
-#undef TLG_EXPERT_CASE
+    const int eg = group_grid(a) + 8 * n;
+    // + 200: streaming stores
+    const int key = ci + ((g_expert_sched >= 0 ? g_expert_sched : dense ? 2 : 1) == 2 ? 200 : 0);
+    if (!tlg_expert_part(key, group_seal(a), eg, st))
+        return tlg_fail(TLG_EINVAL, "expert launch: no kernel for tile form %d", key);
     TLG_HIP(hipGetLastError());
     if (red.nprob && (carry & TLG_ECARRY_OUT) && !dense && g_npending == 0) {
         g_ecarry = red;                  // the next expert launch runs them
@@ -2308,7 +1067,7 @@ int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E,
         g_ecarry_eoff = eoff;
         g_ecarry_st = st;
     } else if (red.nprob) {
-        hipLaunchKernelGGL((k_expert_group<T3>), dim3(group_grid(red)), dim3(T3::THREADS), 0, st, group_seal(red));
+        launch_reductions(red, st);
         TLG_HIP(hipGetLastError());
     }
     return TLG_OK;
