@@ -52,7 +52,7 @@ def reduction(op, M, K, N):
 
 
 # (M, K, N): a tile, stage or chunk ends one short, exactly, or one past
-EDGES = [(9, 16, 16), (32, 32, 32), (33, 20, 68), (64, 15, 64), (65, 17, 63), (127, 48, 129), (128, 128, 128),
+EDGES = [(9, 16, 16), (70, 1, 33), (70, 33, 1), (70, 3, 2), (1030, 2, 5), (9, 130, 3), (67, 261, 254), (32, 32, 32), (33, 20, 68), (64, 15, 64), (65, 17, 63), (127, 48, 129), (128, 128, 128),
          (257, 131, 259), (300, 64, 36), (513, 4, 72), (1024, 512, 192), (2050, 72, 516)]
 
 

@@ -80,7 +80,8 @@ static GemmPlan make_plan(int ci, int Mo, int No, int R, int splits, size_t ws_f
 // Automatic choice: the largest of 128x128, 64x64 and 32x32 tiles that gives
 // the 256 CUs about 160 work items, splitting the reduction as far as every
 // split keeps >= 512 steps (small outputs with long reductions, i.e. mm_atb's
-// dW).  Measured, best other shape against the rule's: mm (8192, 384, 2048)
+// dW), 256 on 32x32 tiles (mm_atb (1001, 77, 333) 9.9 us in 3 splits, 13.6
+// whole).  Measured, best other shape against the rule's: mm (8192, 384, 2048)
 // 128x128 79 us, 128x64 83, 64x64 103; mm (4096, 768, 256) 64x64 14.5,
 // 32x32 20.2; mm (2048, 512, 128) 32x32 7.3, 64x64 10.7; mm_atb
 // (8192, 1024, 384) 8 splits of 128x128 47.5, 64x64 51.4.  64x64 tiles take
@@ -91,7 +92,7 @@ static GemmPlan plan_gemm(int Mo, int No, int R, size_t ws_floats)
 {
     if (g_force_cfg >= 0 && g_force_cfg < kNumCfgs)
         return make_plan(g_force_cfg, Mo, No, R, g_force_splits, ws_floats);
-    const int enough = 160, maxs = R / 512 > 1 ? R / 512 : 1;
+    const int enough = 160;
     const int order[] = {9, R >= 512 ? 8 : 3, 15};
     int ci = 15, splits = 1;
     for (int k = 0; k < 3; k++) {
@@ -99,7 +100,8 @@ static GemmPlan plan_gemm(int Mo, int No, int R, size_t ws_floats)
         const long long tiles = (long long)cdiv(Mo, c.bm) * cdiv(No, c.bn);
         ci = order[k];
         splits = tiles >= enough ? 1 : cdiv(enough, (int)tiles);
-        if (splits > maxs) splits = maxs;
+        const int maxs = R / (k == 2 ? 256 : 512);
+        if (splits > maxs) splits = maxs > 1 ? maxs : 1;
         if (tiles * splits >= enough) break;
     }
     return make_plan(ci, Mo, No, R, splits, ws_floats);

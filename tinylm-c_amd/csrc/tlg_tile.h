@@ -54,6 +54,7 @@
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -128,11 +129,12 @@ struct LdsOp {
     }
 };
 
-// Stage one operand tile into registers.  OUTER = tile extent along the
-// operand's output index.  Tile rows (RC) or columns (OC) past `oext` re-read
+// Stage one operand tile into registers, four values per load (a 16-byte load
+// needs 4-byte alignment only; VEC = the rows themselves are whole float4s).
+// OUTER = tile extent along the operand's output index.  Tile rows (RC) or columns (OC) past `oext` re-read
 // the last valid ones: they feed only outputs that are not stored.  Steps
 // past `rend` (the last stage of a reduction that is no multiple of BK) are
-// read from sixteen zero bytes.
+// read from sixteen zero bytes, or left out value by value without VEC.
 //
 // Two forms serve the expert GEMMs of the MoE layer (float4 path only):
 //   G   gathered rows: the operand's memory row of tile row x is map[x] (RC:
@@ -151,6 +153,9 @@ struct TilePtr {
     static constexpr int PER = OUTER * BK / 4 / NT;   // float4 chunks per thread
     static constexpr int W = PER % 2 == 0 ? 2 : 1;    // neighbouring float4s per chunk of a thread
     static constexpr int HALF = OUTER / 2;
+    // Without VEC an OC row may end inside a chunk: the chunk is then read
+    // ending with the row, and its values move down by this many places.
+    __device__ __forceinline__ int shift(int tid, int q) const { return o0 + col(tid, q) - (oext - 4); }
     // chunk q of thread tid: its row (outer index RC, step OC) and first column
     __device__ static __forceinline__ int row(int tid, int q)
     {
@@ -163,15 +168,15 @@ struct TilePtr {
     static_assert(OUTER * BK / 4 % NT == 0, "tile must split evenly over the workgroup's threads");
     static_assert(!PB || (LAY == OC && HALF % 4 == 0), "paired columns: OC tiles");
     static_assert(!(G || PB) || VEC, "gathered / paired tiles load float4");
-    const float *p[PER];                              // (without VEC: p[0] = the operand)
+    const float *p[PER];
+    const float *P;
     const int *map;
     int ld, o0, oext, rend;
 
-    __device__ __forceinline__ void init(const float *__restrict__ P, int ld_, int o0_, int oext_, int r0, int rend_,
+    __device__ __forceinline__ void init(const float *__restrict__ P_, int ld_, int o0_, int oext_, int r0, int rend_,
                                          int tid, const int *__restrict__ map_, const float *__restrict__ P2)
     {
-        ld = ld_; o0 = o0_; oext = oext_; rend = rend_; map = map_;
-        if (!VEC) { p[0] = P; return; }
+        P = P_; ld = ld_; o0 = o0_; oext = oext_; rend = rend_; map = map_;
 #pragma unroll
         for (int q = 0; q < PER; q++) {
             if (LAY == RC) {
@@ -213,23 +218,38 @@ struct TileLoader {
 #pragma unroll
         for (int q = 0; q < PER; q++) {
             const int pr = Ptr::row(tid, q), pc = Ptr::col(tid, q);
+            const float *p = t.p[q];
+            if constexpr (G && LAY == OC) p += (size_t)rs[q] * t.ld;
+            else p += LAY == RC ? (size_t)dr : (size_t)dr * t.ld;
             if constexpr (VEC) {
-                const float *p = t.p[q];
-                if constexpr (G && LAY == OC) p += (size_t)rs[q] * t.ld;
-                else p += LAY == RC ? (size_t)dr : (size_t)dr * t.ld;
                 if constexpr (TAIL) {
                     if (r0 + (LAY == RC ? pc : pr) >= t.rend) p = g_zero_chunk;
                 }
                 v[q] = *reinterpret_cast<const f32x4 *>(p);
+            } else if constexpr (!TAIL) {
+                v[q] = *reinterpret_cast<const f32x4u *>(p);
             } else {
                 f32x4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    const int o = t.o0 + (LAY == RC ? pr : pc + c);
+                    const int o = min(t.o0 + (LAY == RC ? pr : pc + c), t.oext - 1);
                     const int r = r0 + (LAY == RC ? pc + c : pr);
-                    if (o < t.oext && r < t.rend)
-                        x[c] = LAY == RC ? t.p[0][(size_t)o * t.ld + r] : t.p[0][(size_t)r * t.ld + o];
+                    if (r < t.rend) x[c] = LAY == RC ? t.P[(size_t)o * t.ld + r] : t.P[(size_t)r * t.ld + o];
                 }
+                v[q] = x;
+            }
+        }
+    }
+    // (see TilePtr::shift)
+    __device__ __forceinline__ void align(const Ptr &t, int tid)
+    {
+        if constexpr (!VEC && LAY == OC) {
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                const int s = t.shift(tid, q);
+                f32x4 x = v[q];
+                if (s > 0 && (s & 1)) x = f32x4{x[1], x[2], x[3], x[3]};
+                if (s > 0 && (s & 2)) x = f32x4{x[2], x[3], x[3], x[3]};
                 v[q] = x;
             }
         }
@@ -374,8 +394,11 @@ __device__ __forceinline__ void tile_accumulate(float *__restrict__ smem, const 
     char *lds = reinterpret_cast<char *>(smem);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wm = T::wm(), wn = T::wn(), rb = T::wk() * RW;
-    const int nfull = (rend - rbeg) / BK;             // whole stages; then one with a tail, if any
     if (rend <= rbeg) return;
+    // whole stages; then one with a tail, if any (every stage is taken as one
+    // where rows are shorter than a chunk)
+    const bool narrow = !VEC && ((LA == OC && Mo < 4) || (LB == OC && No < 4));
+    const int nfull = narrow ? 0 : (rend - rbeg) / BK;
 
     // Every prefetch is issued unconditionally: a stage past the end re-reads
     // the last whole stage's (in-bounds) addresses and is never used.  Loads
@@ -432,7 +455,9 @@ __device__ __forceinline__ void tile_accumulate(float *__restrict__ smem, const 
             a.prep(pa, rbeg + stage(st + NR), tid);   // the map rows of its next stage
             b.template load<false>(pb, rbeg + dr, dr, tid);
         };
-        auto put = [&](const LoadA &a, const LoadB &b, int st) {
+        auto put = [&](LoadA &a, LoadB &b, int st) {
+            a.align(pa, tid);
+            b.align(pb, tid);
             char *L = lds + (st & 1) * (SA + SB);
             a.store(L, tid);
             b.store(L + SA, tid);
@@ -466,13 +491,13 @@ __device__ __forceinline__ void tile_accumulate(float *__restrict__ smem, const 
             if (st + k < nfull) step(st + k, k);
         __syncthreads();
     }
-    if (rbeg + nfull * BK < rend) {
+    for (int r0 = rbeg + nfull * BK; r0 < rend; r0 += BK) {
         LoadA a;
         LoadB b;
         Frags f;
-        a.prep(pa, rbeg + nfull * BK, tid);
-        a.template load<true>(pa, rbeg + nfull * BK, nfull * BK, tid);
-        b.template load<true>(pb, rbeg + nfull * BK, nfull * BK, tid);
+        a.prep(pa, r0, tid);
+        a.template load<true>(pa, r0, r0 - rbeg, tid);
+        b.template load<true>(pb, r0, r0 - rbeg, tid);
         a.store(lds, tid);
         b.store(lds + SA, tid);
         __syncthreads();
