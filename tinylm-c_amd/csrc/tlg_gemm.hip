@@ -987,9 +987,10 @@ int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E,
     if (need(rps) > g_tlg.ws_floats)
         return tlg_fail(TLG_ENOMEM, "expert launch: %d experts' partials exceed the workspace", E);
 
-    // tile shape: the largest of 64x64, 64x32 and 32x32 that gives about 320
-    // items (the m3 MoE layer 243 us on 64x64 tiles, 267 on 64x32, 246 on
-    // 128x128, whose SwiGLU epilogue costs the m8 step 1 %)
+    // tile shape: 128x128 (8 waves of 32x64, so a SwiGLU pair shares a lane)
+    // from 160 items on, else the largest of 64x64, 64x32 and 32x32 that gives
+    // about 320 (m8 training step 7.29 ms on 128x128 tiles, 7.64 on 64x64; the
+    // m3 MoE layer 241 us, 243 on 64x64, 267 on 64x32)
     auto items_for = [&](const TileCfg &c) {
         double t = 0;
         for (int i = 0; i < n; i++) {
@@ -1000,6 +1001,7 @@ int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E,
         return t;
     };
     const int ci = g_expert_cfg >= 0 ? g_expert_cfg
+                 : items_for(expert_shape(9)) >= 160 ? 9
                  : items_for(expert_shape(3)) >= 320 ? 3
                  : items_for(expert_shape(14)) >= 320 ? 14 : 15;
     const TileCfg tc = expert_shape(ci);
