@@ -10,7 +10,7 @@ __global__ void k_split_reduce(const float *__restrict__ ws, float *__restrict__
                                int ldc, int splits, int beta)
 {
     const size_t n = (size_t)Mo * No;
-    const size_t per = 256;
+    const size_t per = 512;
     for (size_t e0 = (size_t)blockIdx.x * per; e0 < n; e0 += (size_t)gridDim.x * per)
         reduce_range(ws, C, No, ldc, splits, beta, e0, e0 + per < n ? e0 + per : n, n);
 }
@@ -149,9 +149,9 @@ static int launch_reduce(const float *ws, float *C, int Mo, int No, int ldc, int
                          hipStream_t st)
 {
     const size_t n = (size_t)Mo * No;
-    size_t blocks = (n + 255) / 256;
+    size_t blocks = (n + 511) / 512;
     if (blocks > 2048) blocks = 2048;
-    hipLaunchKernelGGL(k_split_reduce, dim3((unsigned)blocks), dim3(256), 0, st, ws, C, Mo, No, ldc,
+    hipLaunchKernelGGL(k_split_reduce, dim3((unsigned)blocks), dim3(128), 0, st, ws, C, Mo, No, ldc,
                        splits, beta);
     TLG_HIP(hipGetLastError());
     return TLG_OK;
@@ -707,7 +707,7 @@ int tlg_group_launch(const TlgGemmCall *calls, int n, hipStream_t st)
             if (items < row.items) continue;
             if (ci == 33 && !tn) {
                 const double rounds = items / 256.0;
-                if (rounds < 2.0 && rounds / (rounds > 1.0 ? 2.0 : 1.0) < 0.7) continue;
+                if (rounds < (rounds > 1.0 ? 1.7 : 0.7)) continue;
                 if (rounds < 1.0 && rmax <= 512) continue;
                 if (rmax <= 512) ci = 47;
             }
