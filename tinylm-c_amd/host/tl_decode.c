@@ -405,12 +405,13 @@ static int run_chunk(TlDecode *d, int m, int use_state, int start, int copy, voi
 }
 
 /* forward_chunk's layers for m <= bulk prompt rows at positions start.. (all
- * below W, dense layers, no logits): what successive chunks of mmax rows do,
- * with the projections as MFMA GEMMs over all rows instead of one weight
- * stream per chunk.  Rows below W take ring slots of their own, so a row sees
- * the same keys however the prompt is cut.  A 250-token prompt of the
- * 8-layer, D = 384 model took 32 chunks of 0.42 ms. */
-static int run_bulk(TlDecode *d, const int *tok, int m, int start, void *st)
+ * below W, dense layers): what successive chunks of mmax rows do, with the
+ * projections as MFMA GEMMs over all rows instead of one weight stream per
+ * chunk.  Rows below W take ring slots of their own, so a row sees the same
+ * keys however the prompt is cut.  The last `tail` rows go on to the logits,
+ * as the last chunk's; the others end with the last layer's ring.  A 250-token
+ * prompt of the 8-layer, D = 384 model took 32 chunks of 0.42 ms. */
+static int run_bulk(TlDecode *d, const int *tok, int m, int start, int tail, void *st)
 {
     const TlModel *md = &d->m;
     const int D = md->D, H = md->H, KV = md->KV, KD = d->KD, F = md->F, hd = d->hd;
@@ -429,18 +430,24 @@ static int run_bulk(TlDecode *d, const int *tok, int m, int start, void *st)
         CK(tlg_dev_rope(d->bq, d->bpos, 1, m, H, hd, d->rcos, d->rsin, d->maxpos, 0, st));
         CK(tlg_dev_rope(d->bk, d->bpos, 1, m, KV, hd, d->rcos, d->rsin, d->maxpos, 0, st));
         CK(tlg_dev_kv_store(d->bk, d->bv, d->bpos, m, KD, d->W, d->f16, d->Kc[l], d->Vc[l], st));
-        if (l == md->L - 1) break;               /* the last layer's rows feed only its ring */
-        CK(tlg_dev_dec_attn(d->bq, d->Kc[l], d->Vc[l], d->bpos, d->bctx, m, H, KV, hd, d->W, dwin(md, l), d->f16,
-                            d->exact, st));
-        TlgGemmCall o = MMc(y, d->bctx, P + w.wo, m, D, D);
-        o.R = x;
-        CK(tlg_dev_gemm_group(&o, 1, st));
-        CK(tlg_dev_rmsnorm_fwd(y, P + w.an2, d->bn, NULL, m, D, st));
-        CK(tlg_dev_swiglu_mm(d->bn, P + w.w1, P + w.w3, d->bact, NULL, NULL, m, D, F, st));
-        TlgGemmCall f = MMc(x, d->bact, P + w.w2, m, F, D);
-        f.R = y;
-        CK(tlg_dev_gemm_group(&f, 1, st));
+        /* rows [r0, m) go on: past the last layer only the tail's */
+        const int r0 = l == md->L - 1 ? m - tail : 0, mr = m - r0;
+        if (mr == 0) return 0;
+        const size_t o = (size_t)r0 * D;
+        CK(tlg_dev_dec_attn(d->bq + o, d->Kc[l], d->Vc[l], d->bpos + r0, d->bctx + o, mr, H, KV, hd, d->W, dwin(md, l),
+                            d->f16, d->exact, st));
+        TlgGemmCall oc = MMc(y + o, d->bctx + o, P + w.wo, mr, D, D);
+        oc.R = x + o;
+        CK(tlg_dev_gemm_group(&oc, 1, st));
+        CK(tlg_dev_rmsnorm_fwd(y + o, P + w.an2, d->bn + o, NULL, mr, D, st));
+        CK(tlg_dev_swiglu_mm(d->bn + o, P + w.w1, P + w.w3, d->bact + (size_t)r0 * F, NULL, NULL, mr, D, F, st));
+        TlgGemmCall fc = MMc(x + o, d->bact + (size_t)r0 * F, P + w.w2, mr, F, D);
+        fc.R = y + o;
+        CK(tlg_dev_gemm_group(&fc, 1, st));
     }
+    CK(tlg_memcpy_d2d(d->x, x + (size_t)(m - tail) * D, 4 * (size_t)tail * D, st));
+    dmap(d, 0, &w);
+    DGEMV(st, DG(1, 0, d->logits, tail, md->V, D, d->x, P + w.emb, 1, P + w.nf, NULL));
     return 0;
 }
 
@@ -453,21 +460,24 @@ int tl_decode_chunk(TlDecode *d, const int *tok, int m, int start, void *st)
     return run_chunk(d, m, 0, start, 0, st);
 }
 
-/* The leading rows of a prompt through run_bulk: whole chunks of mmax rows
- * that lie below W and leave the last chunk (whose logits and rows the caller
- * reads) to tl_decode_chunk; *done = the rows taken. */
-static int prime_bulk(TlDecode *d, const int *prompt, int n, int *done, void *st)
+/* A prompt's rows through run_bulk: all of them when they fit the ring, else
+ * the whole chunks of mmax rows that lie below W; *done = the rows taken,
+ * *last = the last chunk's rows if it is among them. */
+static int prime_bulk(TlDecode *d, const int *prompt, int n, int *done, int *last, void *st)
 {
-    const int in = (n < d->W ? n : d->W) / d->mmax * d->mmax;
-    const int rows = in < n ? in : n - d->mmax;
+    const int tail = (n - 1) % d->mmax + 1;
+    const int rows = n <= d->W ? n : d->W / d->mmax * d->mmax;
     *done = 0;
-    if (d->unfused || !d->bulk || rows < 2 * TLD_MAXM || n > d->maxpos) return 0;
+    if (d->unfused || !d->bulk || rows - tail < 2 * TLD_MAXM || n > d->maxpos) return 0;
     for (int j = 0; j < rows; j++) if (prompt[j] < 0 || prompt[j] >= d->m.V) return TLG_EINVAL;
-    for (int i = 0; i < rows; i += d->bulk) {
-        const int m = rows - i < d->bulk ? rows - i : d->bulk;
-        CK(run_bulk(d, prompt + i, m, i, st));
+    for (int i = 0, m; i < rows; i += m) {
+        m = rows - i < d->bulk ? rows - i : d->bulk;
+        /* the tail in one piece */
+        if (rows == n && i + m < n && i + m > n - tail) m = n - tail - i;
+        CK(run_bulk(d, prompt + i, m, i, rows == n && i + m == n ? tail : 0, st));
     }
     *done = rows;
+    if (rows == n) *last = tail;
     return 0;
 }
 
@@ -475,7 +485,7 @@ int tl_decode_prime(TlDecode *d, const int *prompt, int n, void *st)
 {
     if (n <= 0) return TLG_EINVAL;
     int i = 0, m = 0;
-    CK(prime_bulk(d, prompt, n, &i, st));
+    CK(prime_bulk(d, prompt, n, &i, &m, st));
     while (i < n) {
         m = n - i < d->mmax ? n - i : d->mmax;
         CK(tl_decode_chunk(d, prompt + i, m, i, st));
@@ -510,7 +520,7 @@ int tl_decode_generate_spec(TlDecode *d, const int *prompt, int np, int n, int *
     if (!d || !prompt || np <= 0 || n <= 0 || !toks || K < 1 || K + 1 > d->mmax || K + 1 > 16) return TLG_EINVAL;
     /* prefill in chunks of mmax (positions 0..np-1), as tl_decode_prime */
     int i = 0, m = 0;
-    CK(prime_bulk(d, prompt, np, &i, st));
+    CK(prime_bulk(d, prompt, np, &i, &m, st));
     while (i < np) {
         m = np - i < d->mmax ? np - i : d->mmax;
         CK(tl_decode_chunk(d, prompt + i, m, i, st));
