@@ -210,7 +210,7 @@ def read_rocprof_avg_us(kernel):
     return None
 
 
-AUTOTUNE_CANDS = (3, 5, 8, 9, 12, 13, 14, 15, 20, 21, 24, 26, 27, 28, 32, 33, 34, 35, 37, 41, 47)
+AUTOTUNE_CANDS = (3, 8, 9, 12, 13, 14, 15, 20, 21, 24, 26, 27, 28, 32, 33, 34, 35, 37, 41, 47)
 # split targets tried with each tile candidate (tlg_tune_group_split: reduction
 # steps per split work item of the mm_atb problems; 0 = the library's rule)
 AUTOTUNE_RTS = (0, 256, 512, 1024, 2048, 4096)
@@ -916,7 +916,7 @@ def main():
     full = None
     if args.full_steps > 0:
         full = bench_full_step(lib, host, stream, args.config, args.full_steps, eager=args.full_eager,
-                               tune=not args.no_autotune)
+                               tune=args.autotune)
         full["gemm_set_share"] = round(ms_step / full["ms_per_step"], 4)
         log(f"[full step] {full}")
     dec_full = None

@@ -373,7 +373,7 @@ extern "C" int tlg_tune_group_policy(const int *cands, int ncands, double min_wa
     if (ncands < 0 || ncands > 3 || (ncands > 0 && !cands) || min_waves < 0 || (rtarget && rtarget < 64))
         return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: bad arguments");
     for (int k = 0; k < ncands; k++)
-        if (cands[k] < 0 || cands[k] >= kNumCfgs)
+        if (cands[k] < 0 || cands[k] >= kNumCfgs || cands[k] == 2 || (cands[k] >= 5 && cands[k] <= 7))
             return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: config %d", cands[k]);
     if (ncands > 0) {
         for (int k = 0; k < ncands; k++) g_cand[k] = cands[k];
@@ -396,7 +396,7 @@ extern "C" int tlg_tune_expert(int cfg, int sched)
 
 extern "C" int tlg_tune_group(int cfg)
 {
-    if (cfg < -1 || cfg >= kNumCfgs)
+    if (cfg != -1 && cfg != 0 && cfg != 1 && cfg != 3 && cfg != 4 && (cfg < 8 || cfg >= kNumCfgs))
         return tlg_fail(TLG_EINVAL, "tlg_tune_group: config %d", cfg);
     g_group_cfg = cfg;
     return TLG_OK;
