@@ -237,6 +237,33 @@ def test_bench_tables_match_oracle(lib, orc, name):
             assert normwise_rel(got[bname][a:b], init[bname][a:b]) <= TOL, (name, label)
 
 
+@pytest.mark.parametrize("cfgs", [(3, 21, 33), (15, 34, 14)], ids=str)
+def test_launches_keep_their_kernel_names(lib, cfgs):
+    """tl_run_launch_kernel(k) names launch k's own kernel, whatever ran after
+    it, and a pointer from tlg_group_kernel outlives later launches."""
+    host = tlgemm.host()
+    plan = host.plan_train(**bench.TRAIN["nano"])
+    run, stream = new_run(lib, host, plan, seed=3)
+    want = {3: "64, 64, 16, ", 21: "64, 32, 64, ", 33: "128, 128, 16, ", 15: "32, 32, 64, ", 34: "128, 64, 32, ",
+            14: "64, 32, 32, "}
+    try:
+        L = host.dll.tl_run_grouped_launches(run)
+        for k in range(L):
+            assert host.dll.tl_run_set_launch_config(run, k, cfgs[k % 3]) == 0
+        ev = (ctypes.c_void_p * (L + 2))(*[lib.tlg_event_create() for _ in range(L + 2)])
+        lib.check(host.dll.tl_run_time_launches(run, ev, L + 2, stream), "step")
+        names = [host.dll.tl_run_launch_kernel(run, k) for k in range(L)]
+        lib.check(lib.tlg_stream_sync(stream), "sync")
+        for e in ev:
+            lib.tlg_event_destroy(e)
+    finally:
+        host.dll.tl_run_free(run)
+    named = [(k, n.decode()) for k, n in enumerate(names) if n and n.startswith(b"k_group<")]
+    assert {k % 3 for k, _ in named} == {0, 1, 2}
+    for k, n in named:
+        assert "Tile<" + want[cfgs[k % 3]] in n, (k, n)
+
+
 def test_split_target_hook_rejects_small_targets(lib):
     assert lib.tlg_tune_group_split(63) != 0
     assert lib.tlg_tune_group_split(0) == 0

@@ -3,6 +3,8 @@
 // and expert-batched launches, the fills and the measurement probes.
 #include "tlg_tile.h"
 #include <mutex>
+#include <set>
+#include <string>
 #include <stdio.h>
 #include <string.h>
 
@@ -410,14 +412,21 @@ extern "C" int tlg_tune_group_split(int rtarget)
     return TLG_OK;
 }
 
+// Callers keep the pointer past later launches, so each name is stored once
+// (at most one string per kernel instance) and never rewritten.
 const char *tlg_group_kernel_name(void)
 {
-    if (g_group_last_name) return g_group_last_name;
-    static char name[128];
-    char tile[96];
-    tile_name(kCfgs[g_group_last], tile, (int)sizeof tile);
-    snprintf(name, sizeof name, "k_group<%s >", tile);
-    return name;
+    static std::set<std::string> names;
+    static std::mutex mu;
+    char name[128], tile[96];
+    if (g_group_last_name) {
+        snprintf(name, sizeof name, "%s", g_group_last_name);
+    } else {
+        tile_name(kCfgs[g_group_last], tile, (int)sizeof tile);
+        snprintf(name, sizeof name, "k_group<%s >", tile);
+    }
+    std::lock_guard<std::mutex> lk(mu);
+    return names.insert(name).first->c_str();
 }
 
 // Grid for the XCD-sliced mapping of group_item: 8 x the largest per-XCD
