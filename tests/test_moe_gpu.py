@@ -256,6 +256,41 @@ def test_expert_tile_forms(lib, orc, cfg, sched):
     assert lib.tlg_tune_expert(8, 1) != 0 and lib.tlg_tune_expert(3, 3) != 0
 
 
+@pytest.mark.parametrize("cfg", [-1, 3, 14, 15, 18, 22])
+@pytest.mark.parametrize("dims", [(300, 132, 196, 3), (67, 32, 48, 3)], ids=str)
+def test_operands_without_a_split(lib, cfg, dims):
+    """Infinities, NaN and a weight that rounds to bf16's infinity in the expert
+    weights, an infinite and a NaN output gradient: the outputs they enter are
+    NaN or infinite where fp64's are and the others stay within the bar, on
+    every expert tile shape (column pairs, gathered rows, the gathered dW sums)."""
+    N, D, F, E = dims
+    c = case(N, D, F, E, zlib.crc32(f"moe inf {dims}".encode()))
+    c["w3"][1, 2, 5], c["w2"][2, 7, 3], c["w1"][0, 4, 9] = np.inf, np.nan, np.float32(-3.4e38)
+    c["fnorm"][:, 4] = np.clip(c["fnorm"][:, 4], -0.4, 0.4)       # g and g u stay in fp32's range
+    lib.check(lib.tlg_tune_expert(cfg, -1), "tune expert")
+    try:
+        out, assign, gate, rprobs = gpu_forward(lib, c["fnorm"], c["fin"], c["wr"], c["w1"], c["w3"], c["w2"])
+        assert set(assign) == set(range(E))
+        c["dout"][np.nonzero(assign == 0)[0][3], 6] = np.inf
+        c["dout"][np.nonzero(assign == 1)[0][1], 2] = np.nan
+        zero = [np.zeros_like(c[k]) for k in ("gwr0", "gw10", "gw30", "gw20")]
+        dfn, grads = gpu_backward(lib, c["fnorm"], c["dout"], assign, gate, rprobs, c["wr"], c["w1"], c["w3"],
+                                  c["w2"], *zero)
+    finally:
+        lib.check(lib.tlg_tune_expert(-1, -1), "tune expert")
+    with np.errstate(all="ignore"):
+        o64, dfn64, _, *g64 = f64_moe(c["fnorm"], c["fin"], c["wr"], c["w1"], c["w3"], c["w2"], c["dout"], assign)
+    for name, got, ref in zip(("out", "dfn", "gw1", "gw3", "gw2"), [out, dfn] + grads[1:], [o64, dfn64] + g64):
+        wild = ~np.isfinite(ref) | (np.abs(ref) > 3e38)
+        assert np.array_equal(np.isfinite(got), ~wild), (name, np.argwhere(np.isfinite(got) == wild)[:4])
+        inf = np.isinf(ref)
+        assert np.array_equal(got[inf], ref[inf].astype(np.float32)), name
+        # the 3.4e38 weight makes ordinary values of up to 1e38 beside ordinary ones
+        fine = ~wild & (np.abs(ref) < 1e6)
+        scale = np.maximum(np.abs(ref[fine]), np.median(np.abs(ref[fine])))
+        assert fine.mean() > 0.1 and (np.abs(got[fine] - ref[fine]) <= TOL * scale).all(), name
+
+
 def test_skewed_split(lib):
     """The skewed config really is unbalanced (so the test above exercises
     experts of very different row counts)."""

@@ -2,6 +2,8 @@
 products of them on the matrix cores.  Error against fp64, operands that have
 no such split (infinities, NaN, magnitudes past bf16's largest), and the
 sizes where a tile, a stage or a chunk ends."""
+import contextlib
+
 import numpy as np
 import pytest
 
@@ -85,6 +87,10 @@ def test_error_against_fp64(lib, op, shape):
 def test_operands_without_a_split(lib, op, grouped, shape):
     """Infinities, NaN and values that round to bf16's infinity give what fp32
     sums give, and leave the outputs they do not enter alone."""
+    check_without_a_split(lib, op, grouped, shape)
+
+
+def check_without_a_split(lib, op, grouped, shape):
     M, K, N = shape
     r = np.random.default_rng(3)
     X = r.standard_normal((M, K), dtype=np.float32)
@@ -116,3 +122,62 @@ def test_magnitudes(lib, scale):
     W = (r.standard_normal((80, 112)) / (scale if scale > 1 else 1)).astype(np.float32)
     got, ref = run(lib, "mm", X, W, W[:1], False), want("mm", X, W, W[:1])
     assert np.linalg.norm(got - ref) <= 4 * 2.0 ** -24 * (1 + np.sqrt(5)) * np.linalg.norm(ref)
+
+
+# every shape of the automatic rules, pinned: single calls whole and split,
+# grouped launches (128x128, 128x64, 64x64, 64x32 and 32x32 tiles, wave groups
+# along the reduction and none)
+PINNED = [(False, c, sp) for c in (9, 8, 3, 15) for sp in (1, 3)] + [(True, c, 0) for c in (33, 47, 34, 35, 41, 21, 15)]
+
+
+@contextlib.contextmanager
+def pinned(lib, grouped, cfg, splits):
+    lib.check(lib.tlg_tune_group(cfg) if grouped else lib.tlg_tune_force(cfg, splits), "pin")
+    try:
+        yield
+    finally:
+        lib.check(lib.tlg_tune_group(-1) if grouped else lib.tlg_tune_force(-1, 0), "unpin")
+
+
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+@pytest.mark.parametrize("pin", PINNED, ids=str)
+def test_operands_without_a_split_on_every_shape(lib, op, pin):
+    """The same on each tile shape, at ragged sizes past one and two of the
+    largest tiles (aligned rows, and odd ones for the single calls)."""
+    for shape in ((200, 132, 260), (304, 260, 132)) + (() if pin[0] else ((201, 131, 259),)):
+        with pinned(lib, *pin):
+            check_without_a_split(lib, op, pin[0], shape)
+
+
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+def test_a_nan_does_not_stall_the_launch(lib, op):
+    """One NaN in each operand sends a row and a column of outputs, and NaN
+    weights every output, through the fp32 sums.  On the matrix cores that takes 2
+    to 5 times the finite call (one lane per output took 25 to 80 times)."""
+    torch = _torch()
+    M, K, N = 4096, 256, 768
+    X, W, dY = (torch.randn(*s, device="cuda") for s in ((M, K), (K, N), (M, N)))
+    a, b, out = {"mm": (X, W, torch.zeros(M, N, device="cuda")), "mm_bt": (dY, W, torch.zeros(M, K, device="cuda")),
+                 "mm_atb": (X, dY, torch.zeros(K, N, device="cuda"))}[op]
+    f = {"mm": lib.mm, "mm_bt": lib.mm_bt, "mm_atb": lib.mm_atb}[op]
+    st = torch.cuda.current_stream().cuda_stream
+
+    def us():
+        best = 1e9
+        for _ in range(5):
+            e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            e0.record()
+            for _ in range(5):
+                f(out.data_ptr(), a.data_ptr(), b.data_ptr(), M, K, N, st)
+            e1.record()
+            torch.cuda.synchronize()
+            best = min(best, 200 * e0.elapsed_time(e1))
+        return best
+
+    finite = us()
+    a[5, 7] = b[3, 5] = float("nan")
+    one = us()
+    b[:] = float("nan")
+    every = us()
+    print(op, "finite", finite, "one NaN", one, "all", every, flush=True)
+    assert max(one, every) <= 12 * finite, (finite, one, every)

@@ -489,9 +489,18 @@ __device__ __forceinline__ void tile_accumulate(float *__restrict__ smem, const 
 #pragma unroll
             for (int k = 0; k < NR; k++) step(st + k, k);
         }
+        // The sums stay in their registers here: one-block waves copied all of
+        // them at the end of every turn (33 moves behind the last MFMA).
+#pragma unroll
+        for (int n = 0; n < T::FM * T::FN * T::NCH; n++)
+            asm("" : "+v"(acc[n / T::NCH / T::FN][n / T::NCH % T::FN][n % T::NCH]));
 #pragma unroll
         for (int k = 0; k < NR - 1; k++)
             if (st + k < nfull) step(st + k, k);
+        // The loads past the end have come in: left outstanding, each store of
+        // an epilogue that takes their registers would wait for them, and with
+        // them for the store before it.
+        __builtin_amdgcn_s_waitcnt(0x0f70);           // vmcnt(0)
         __syncthreads();
     }
     for (int r0 = rbeg + nfull * BK; r0 < rend; r0 += BK) {
@@ -510,60 +519,93 @@ __device__ __forceinline__ void tile_accumulate(float *__restrict__ smem, const 
     }
 }
 
-// One segment's share of an output that this wave owns, in plain fp32: steps
-// [rbeg, rend) as the wave's reduction group takes them (RW of each BK).  GA:
-// A's reduction rows go through the map.
-template <class T, int LA, int LB, bool GA = false>
-__device__ __forceinline__ float slow_dot(const float *__restrict__ A, const float *__restrict__ B, int lda, int ldb,
-                                          int i, int j0, int jt, int rbeg, int rend, float s,
-                                          const int *__restrict__ amap = nullptr)
+// One segment's share of a 32x32 block that this wave owns, in plain fp32 on
+// the fp32 matrix cores, operands straight from memory: steps [rbeg, rend) as
+// the wave's reduction group takes them (RW of each BK), eight MFMAs of two
+// steps per sixteen.  pa / pb: this lane's output index of A / B (lane & 31),
+// at step 0.  GA: A's reduction rows go through the map.  Operands are taken
+// times `scale`.
+template <int LAY>
+__device__ __forceinline__ const float *lane_base(const float *P, int o, int ld)
 {
-    const int j = j0 + jt;
-    for (int r0 = rbeg + T::wk() * T::RW; r0 < rend; r0 += T::BK)
-        for (int r = r0; r < min(r0 + T::RW, rend); r++) {
-            const float a = LA == RC ? A[(size_t)i * lda + r] : A[(size_t)(GA ? amap[r] : r) * lda + i];
-            const float b = LB == RC ? B[(size_t)j * ldb + r] : B[(size_t)r * ldb + j];
-            s = fmaf(a, b, s);
+    return LAY == RC ? P + (size_t)o * ld : P + o;
+}
+template <class T, int LA, int LB, bool GA = false>
+__device__ __forceinline__ void fp32_block(f32x16 &c, const float *__restrict__ pa, const float *__restrict__ pb,
+                                           int lda, int ldb, int rbeg, int rend, float scale,
+                                           const int *__restrict__ amap = nullptr)
+{
+    const int h8 = 8 * ((threadIdx.x & 63) >> 5);
+    auto at_a = [&](int r) { return (LA == RC ? pa[r] : pa[(size_t)(GA ? amap[r] : r) * lda]) * scale; };
+    auto at_b = [&](int r) { return (LB == RC ? pb[r] : pb[(size_t)r * ldb]) * scale; };
+#pragma nounroll
+    for (int r0 = rbeg + T::wk() * T::RW; r0 < rend; r0 += T::BK) {
+        float a[8], b[8];
+        const int r = r0 + h8;
+        if (r0 + T::RW <= rend) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) a[k] = at_a(r + k), b[k] = at_b(r + k);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const int rc = min(r + k, rend - 1);
+                a[k] = at_a(rc);
+                b[k] = at_b(rc);
+                if (r + k >= rend) a[k] = b[k] = 0.f;
+            }
         }
-    return s;
+#pragma unroll
+        for (int k = 0; k < 8; k++) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k], b[k], c, 0, 0, 0);
+    }
 }
 
 // Outputs that came out infinite or NaN, again in plain fp32.  An operand that
 // is not finite (or rounds to bf16's infinity) has no split: its pieces turn
 // every sum they enter into NaN where fp32 has infinities, or finite sums of
-// products past the pieces' range.  sum(i, jt): the output at row i and tile
-// column jt.  No wave waits for another here, and finite tiles only look.
-template <class T, bool PB, class Sum>
-__device__ __forceinline__ void tile_fix(f32x16 (&acc)[T::FM][T::FN][T::NCH], int i0, int j0, int Mo, int No, Sum sum)
+// products past the pieces' range.  block(c, i, jt, scale): c += scale^2 times
+// the wave's share of the 32x32 block in which this lane's rows of A and B are
+// row i and tile column jt.  What is still not finite is summed once more at
+// 2^-140: the fp32 MFMA rounds a product that is out of range to infinity, and
+// two of them that cancel to NaN.  No wave waits for another here, and finite
+// tiles only look.
+// 8192 x 384 x 2048, fwd / dX / dW us: finite 81 / 99 / 95; one NaN in each
+// operand 200 / 403 / 570, NaN everywhere 410 / 510 / 646 (one lane per output,
+// 1436 / 4839 / 8101 and 5348 / 15192 / 17235).
+template <class T, class Block>
+__device__ __forceinline__ void tile_fix(f32x16 (&sum)[T::FM][T::FN], int i0, int Mo, Block block)
 {
-    float z = 0.f;                                    // NaN if any sum is not finite
+    auto finite = [](float x) { return fabsf(x) <= 3.402823466e38f; };
+    unsigned need = 0;                                // blocks with a sum that is not finite
 #pragma unroll
-    for (int a = 0; a < T::FM; a++)
+    for (int n = 0; n < T::FM * T::FN; n++) {
+        float z = 0.f;                                // NaN if any is not
 #pragma unroll
-        for (int b = 0; b < T::FN; b++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) z = fmaf(acc[a][b][0][v] + acc[a][b][1][v], 0.f, z);
-    if (!__any(z != z)) return;
-    const int lane = threadIdx.x & 63;
+        for (int v = 0; v < 16; v++) z = fmaf(sum[n / T::FN][n % T::FN][v], 0.f, z);
+        if (__any(z != z)) need |= 1u << n;
+    }
+    if (!need) return;
+    const int o = threadIdx.x & 31;
 #pragma nounroll
-    for (int n = 0; n < T::FM * T::FN * 16; n++) {
-        const int a = n / (T::FN * 16), b = n / 16 % T::FN, v = n % 16;
-        const int i = i0 + T::wm() * T::WM + a * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        const int jt = T::wn() * T::WN + b * 32 + (lane & 31);
-        const int jo = j0 + (PB ? jt / (2 * pair_unit(T::BN)) * pair_unit(T::BN) + jt % pair_unit(T::BN) : jt);
-        if (i >= Mo || jo >= No) continue;
-        float x = 0.f;
+    for (int n = 0; n < T::FM * T::FN; n++) {
+        if (!(need >> n & 1u)) continue;
+        const int i = min(i0 + T::wm() * T::WM + n / T::FN * 32 + o, Mo - 1), jt = T::wn() * T::WN + n % T::FN * 32 + o;
+#pragma nounroll
+        for (float scale = 1.f, back = 1.f;; scale = 0x1p-70f, back = 0x1p70f) {
+            f32x16 c = {};
+            block(c, i, jt, scale);
+            bool wild = false;
 #pragma unroll
-        for (int k = 0; k < T::FM * T::FN * 16; k++)
-            if (k == n) x = acc[k / (T::FN * 16)][k / 16 % T::FN][0][k % 16] + acc[k / (T::FN * 16)][k / 16 % T::FN][1][k % 16];
-        if (fabsf(x) <= 3.402823466e38f) continue;    // finite
-        x = sum(i, jt);
+            for (int k = 0; k < T::FM * T::FN; k++)
+                if (k == n) {
+                    auto &x = sum[k / T::FN][k % T::FN];
 #pragma unroll
-        for (int k = 0; k < T::FM * T::FN * 16; k++)
-            if (k == n) {
-                acc[k / (T::FN * 16)][k / 16 % T::FN][0][k % 16] = x;
-                acc[k / (T::FN * 16)][k / 16 % T::FN][1][k % 16] = 0.f;
-            }
+                    for (int v = 0; v < 16; v++) {
+                        if (!finite(x[v])) x[v] = c[v] * back * back;
+                        wild |= !finite(x[v]);
+                    }
+                }
+            if (back > 1.f || !__any(wild)) break;
+        }
     }
 }
 
@@ -586,16 +628,11 @@ struct NoPre {
     __device__ __forceinline__ E operator()(int, int) const { return E{}; }
 };
 template <class T, bool STASH = false, class Pre, class Put>
-__device__ __forceinline__ void tile_epi(const f32x16 (&accs)[T::FM][T::FN][T::NCH], int Mo, int No, int i0,
-                                         int j0, float *__restrict__ red, Pre pre, Put put)
+__device__ __forceinline__ void tile_epi(const f32x16 (&acc)[T::FM][T::FN], int Mo, int No, int i0, int j0,
+                                         float *__restrict__ red, Pre pre, Put put)
 {
     const int lane = threadIdx.x & 63;
     using E = decltype(pre(0, 0));
-    f32x16 acc[T::FM][T::FN];
-#pragma unroll
-    for (int a = 0; a < T::FM; a++)
-#pragma unroll
-        for (int b = 0; b < T::FN; b++) acc[a][b] = accs[a][b][0] + accs[a][b][1];
     if constexpr (T::WK == 1) {
         const int wm = T::wm(), wn = T::wn();
         const int h = lane >> 5, col = lane & 31;
@@ -617,6 +654,10 @@ __device__ __forceinline__ void tile_epi(const f32x16 (&accs)[T::FM][T::FN][T::N
                 E e[16];
 #pragma unroll
                 for (int v = 0; v < 16; v++) e[v] = pre(min(ib + 8 * (v >> 2) + (v & 3), Mo - 1), min(j, No - 1));
+                // all in: else a path of the kernel that reads nothing would
+                // wait before each of its stores for these registers, and so
+                // for the store before it (64x64 mm 14.4 -> 15.7 us)
+                if constexpr (!__is_empty(E)) __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0)
                 if (j >= No) continue;
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
@@ -678,15 +719,14 @@ __device__ __forceinline__ void st_out(float *p, float v)
 
 // C (beta ? += : =) acc for the valid part of the tile.
 template <class T>
-__device__ __forceinline__ void tile_store(const f32x16 (&accs)[T::FM][T::FN][T::NCH], float *__restrict__ C,
-                                           int ldc, int beta, int Mo, int No, int i0, int j0,
-                                           float *__restrict__ red)
+__device__ __forceinline__ void tile_store(const f32x16 (&acc)[T::FM][T::FN], float *__restrict__ C, int ldc, int beta,
+                                           int Mo, int No, int i0, int j0, float *__restrict__ red)
 {
     if (beta)
-        tile_epi<T>(accs, Mo, No, i0, j0, red, [&](int i, int j) { return C[(size_t)i * ldc + j]; },
+        tile_epi<T>(acc, Mo, No, i0, j0, red, [&](int i, int j) { return C[(size_t)i * ldc + j]; },
                     [&](int i, int j, float v, float c) { st_out<T>(C + (size_t)i * ldc + j, c + v); });
     else
-        tile_epi<T>(accs, Mo, No, i0, j0, red, NoPre(),
+        tile_epi<T>(acc, Mo, No, i0, j0, red, NoPre(),
                     [&](int i, int j, float v, NoPre::E) { st_out<T>(C + (size_t)i * ldc + j, v); });
 }
 
@@ -699,12 +739,12 @@ __device__ __forceinline__ void tile_store(const f32x16 (&accs)[T::FM][T::FN][T:
 // fma chains, then their sum.  Needs No % 32 == 0 and TILE <= the LDS the
 // tile's stages use (every shape but the 128 x 128 ones; the host checks).
 template <class T>
-__device__ __forceinline__ void tile_store_dot(const f32x16 (&accs)[T::FM][T::FN][T::NCH], float *__restrict__ C,
-                                               int ldc, int Mo, int No, int i0, int j0, const float *__restrict__ O,
+__device__ __forceinline__ void tile_store_dot(const f32x16 (&acc)[T::FM][T::FN], float *__restrict__ C, int ldc, int Mo,
+                                               int No, int i0, int j0, const float *__restrict__ O,
                                                float *__restrict__ out, float *__restrict__ red)
 {
     if constexpr (T::TILE <= T::lds_max()) {
-        tile_epi<T, true>(accs, Mo, No, i0, j0, red, NoPre(),
+        tile_epi<T, true>(acc, Mo, No, i0, j0, red, NoPre(),
                           [&](int i, int j, float v, NoPre::E) { st_out<T>(C + (size_t)i * ldc + j, v); });
         __syncthreads();
         // eight lanes per (row, block), lane q holding float4 q of the block
@@ -771,7 +811,7 @@ __host__ __device__ constexpr int expert_lds()
 // registers the launch can run 128x128 tiles: m8 training step 7.64 -> 7.29
 // ms, m3 1.905 -> 1.84 ms, both with the epilogues' reads issued together.
 template <class T>
-__device__ __forceinline__ void tile_swiglu(const f32x16 (&accs)[T::FM][T::FN][T::NCH], float *__restrict__ Ca,
+__device__ __forceinline__ void tile_swiglu(const f32x16 (&acc)[T::FM][T::FN], float *__restrict__ Ca,
                                             float *__restrict__ Cg, float *__restrict__ Cu, int ldc, int Mo,
                                             int No, int i0, int jh, float *__restrict__ red)
 {
@@ -792,14 +832,13 @@ __device__ __forceinline__ void tile_swiglu(const f32x16 (&accs)[T::FM][T::FN][T
 #pragma unroll
                 for (int v = 0; v < 16; v++)
                     emit(i0 + T::wm() * T::WM + a * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3),
-                         jh + (T::wn() * T::WN + b * 32) / 2 + (lane & 31), accs[a][b][0][v] + accs[a][b][1][v],
-                         accs[a][b + 1][0][v] + accs[a][b + 1][1][v]);
+                         jh + (T::wn() * T::WN + b * 32) / 2 + (lane & 31), acc[a][b][v], acc[a][b + 1][v]);
     } else {
         constexpr int H = T::BN / 2, LD = T::BN + 1;
         constexpr int OFF = T::WK > 1 ? T::WK * T::TILE : 0;
         static_assert(OFF + T::BM * LD <= expert_lds<T>(), "paired tile fits beside the partials");
         float *L = red + OFF;
-        tile_epi<T>(accs, T::BM, T::BN, 0, 0, red, NoPre(),
+        tile_epi<T>(acc, T::BM, T::BN, 0, 0, red, NoPre(),
                     [&](int i, int j, float v, NoPre::E) { L[i * LD + j] = v; });
         __syncthreads();
         for (int f = threadIdx.x; f < T::BM * H; f += T::THREADS) {
@@ -808,6 +847,16 @@ __device__ __forceinline__ void tile_swiglu(const f32x16 (&accs)[T::FM][T::FN][T
         }
         __syncthreads();
     }
+}
+
+// The tile's sums: what the large products' and the small ones' accumulators hold.
+template <class T>
+__device__ __forceinline__ void tile_sum(const f32x16 (&acc)[T::FM][T::FN][T::NCH], f32x16 (&sum)[T::FM][T::FN])
+{
+#pragma unroll
+    for (int a = 0; a < T::FM; a++)
+#pragma unroll
+        for (int b = 0; b < T::FN; b++) sum[a][b] = acc[a][b][0] + acc[a][b][1];
 }
 
 template <int FM, int FN, int NCH>
@@ -847,17 +896,19 @@ __global__ __launch_bounds__(T::THREADS) void k_gemm(GemmArgs g)
     const int i0 = (tile / g.tiles_n) * T::BM, j0 = (tile % g.tiles_n) * T::BN;
     const int rbeg = z * g.rps;
     const int rend = min(g.R, rbeg + g.rps);
-    f32x16 acc[T::FM][T::FN][T::NCH];
+    f32x16 acc[T::FM][T::FN][T::NCH], sum[T::FM][T::FN];
     zero_acc(acc);
     tile_accumulate<T, LA, LB, VEC>(smem, g.A, g.B, g.lda, g.ldb, i0, j0, g.Mo, g.No, rbeg, rend, acc);
-    tile_fix<T, false>(acc, i0, j0, g.Mo, g.No, [&](int i, int jt) {
-        return slow_dot<T, LA, LB>(g.A, g.B, g.lda, g.ldb, i, j0, jt, rbeg, rend, 0.f);
+    tile_sum<T>(acc, sum);
+    tile_fix<T>(sum, i0, g.Mo, [&](f32x16 &c, int i, int jt, float scale) {
+        fp32_block<T, LA, LB>(c, lane_base<LA>(g.A, i, g.lda), lane_base<LB>(g.B, min(j0 + jt, g.No - 1), g.ldb),
+                              g.lda, g.ldb, rbeg, rend, scale);
     });
     // a split writes its partial (beta 0) into workspace slice z
     if (g.splits > 1)
-        tile_store<T>(acc, g.ws + (size_t)z * g.Mo * g.No, g.No, 0, g.Mo, g.No, i0, j0, smem);
+        tile_store<T>(sum, g.ws + (size_t)z * g.Mo * g.No, g.No, 0, g.Mo, g.No, i0, j0, smem);
     else
-        tile_store<T>(acc, g.C, g.ldc, g.beta, g.Mo, g.No, i0, j0, smem);
+        tile_store<T>(sum, g.C, g.ldc, g.beta, g.Mo, g.No, i0, j0, smem);
 }
 
 // C (beta ? += : =) sum_{z < splits} ws[z], in z order; Mo x No elements, the
@@ -1012,7 +1063,7 @@ __device__ __forceinline__ void expert_acc(float *smem, const Prob &P, const Seg
 template <class T, int LA, int LB>
 __device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int local, const int *eo)
 {
-    f32x16 acc[T::FM][T::FN][T::NCH];
+    f32x16 acc[T::FM][T::FN][T::NCH], sum[T::FM][T::FN];
     int e, t, base, rows, slot0;
     if (P.kind != PK_TN) {
         if (!expert_of(P, eo, local / P.tiles_n, &e, &t, &base, &rows, &slot0)) return;
@@ -1038,34 +1089,31 @@ __device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int loca
             expert_acc<T, LA, LB>(smem, P, s, A, s.B + (size_t)e * P.es, amap, i0, j0, rows, P.No, 0, s.R,
                                   acc);
         }
-        auto again = [&](int i, int jt) {
-            float x = 0.f;
+        tile_sum<T>(acc, sum);
+        tile_fix<T>(sum, i0, rows, [&](f32x16 &c, int i, int jt, float scale) {
+            // a paired tile's columns alternate between B and B2 (TilePtr PB)
+            const bool pair = LA == RC && LB == OC && P.B2;
+            constexpr int U = pair_unit(T::BN);
+            const int j = min(j0 + (pair ? jt / (2 * U) * U + jt % U : jt), P.No - 1);
             const int am = P.amap ? P.amap[base + i] : base + i;
             for (int k = 0; k < P.nseg; k++) {
                 const Seg &s = P.seg[k];
-                const float *B = s.B + (size_t)e * P.es;
-                constexpr int U = pair_unit(T::BN);
-                if (LA == RC && LB == OC && P.B2)
-                    x = slow_dot<T, LA, LB>(s.A, jt & U ? P.B2 + (B - s.B) : B, s.lda, s.ldb, am, j0,
-                                            jt / (2 * U) * U + jt % U, 0, s.R, x);
-                else
-                    x = slow_dot<T, LA, LB>(s.A, B, s.lda, s.ldb, am, j0, jt, 0, s.R, x);
+                const float *B = (pair && (jt & U) ? P.B2 : s.B) + (size_t)e * P.es;
+                fp32_block<T, LA, LB>(c, lane_base<LA>(s.A, am, s.lda), lane_base<LB>(B, j, s.ldb), s.lda, s.ldb, 0,
+                                      s.R, scale);
             }
-            return x;
-        };
-        if (LA == RC && LB == OC && P.B2) tile_fix<T, true>(acc, i0, j0, rows, P.No, again);
-        else                              tile_fix<T, false>(acc, i0, j0, rows, P.No, again);
+        });
         const size_t cb = (size_t)base * P.ldc;
         switch (P.epi) {
         case TLG_EPI_SWIGLU:
-            tile_swiglu<T>(acc, P.C + cb, P.X1 ? P.X1 + cb : nullptr, P.X2 ? P.X2 + cb : nullptr, P.ldc, rows,
+            tile_swiglu<T>(sum, P.C + cb, P.X1 ? P.X1 + cb : nullptr, P.X2 ? P.X2 + cb : nullptr, P.ldc, rows,
                            P.No, i0, j0, smem);
             break;
         case TLG_EPI_SWIGLU_BWD: {
             // In place: g <- da u silu'(g), u <- da silu(g)  (tinylm.c:923-925)
             float *G = P.X1 + cb, *U = P.X2 + cb;
             const int ld = P.ldc;
-            tile_epi<T>(acc, rows, P.No, i0, j0, smem,
+            tile_epi<T>(sum, rows, P.No, i0, j0, smem,
                         [&](int i, int j) {
                             const size_t o = (size_t)i * ld + j;
                             return f32x2{G[o], U[o]};
@@ -1088,7 +1136,7 @@ __device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int loca
                 float *C = P.C;
                 const float *fin = P.fin;
                 float *Y = P.X1 ? P.X1 + cb : nullptr;      // the expert rows too, when kept
-                tile_epi<T>(acc, rows, P.No, i0, j0, smem,
+                tile_epi<T>(sum, rows, P.No, i0, j0, smem,
                             [&](int i, int j) { return fin[(size_t)s_tok[i - i0] * ld + j]; },
                             [&](int i, int j, float y, float x0) {
                                 const int x = i - i0;
@@ -1099,7 +1147,7 @@ __device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int loca
             break;
         }
         default:
-            tile_store<T>(acc, P.C + cb, P.ldc, P.beta, rows, P.No, i0, j0, smem);
+            tile_store<T>(sum, P.C + cb, P.ldc, P.beta, rows, P.No, i0, j0, smem);
         }
     } else {
         if (!expert_of(P, eo, local / P.tiles, &e, &t, &base, &rows, &slot0)) return;
@@ -1110,11 +1158,13 @@ __device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int loca
         zero_acc(acc);
         // A's reduction rows are sorted rows; gathered ones map through amap
         expert_acc<T, LA, LB>(smem, P, s, s.A, s.B, P.amap, i0, j0, P.Mo, P.No, rbeg, rend, acc);
-        tile_fix<T, false>(acc, i0, j0, P.Mo, P.No, [&](int i, int jt) {
-            return P.amap ? slow_dot<T, LA, LB, true>(s.A, s.B, s.lda, s.ldb, i, j0, jt, rbeg, rend, 0.f, P.amap)
-                          : slow_dot<T, LA, LB>(s.A, s.B, s.lda, s.ldb, i, j0, jt, rbeg, rend, 0.f);
+        tile_sum<T>(acc, sum);
+        tile_fix<T>(sum, i0, P.Mo, [&](f32x16 &c, int i, int jt, float scale) {
+            const float *pa = lane_base<LA>(s.A, i, s.lda), *pb = lane_base<LB>(s.B, min(j0 + jt, P.No - 1), s.ldb);
+            if (P.amap) fp32_block<T, LA, LB, true>(c, pa, pb, s.lda, s.ldb, rbeg, rend, scale, P.amap);
+            else        fp32_block<T, LA, LB>(c, pa, pb, s.lda, s.ldb, rbeg, rend, scale);
         });
-        tile_store<T>(acc, (float *)P.ws + (size_t)(slot0 + t) * P.Mo * P.No, P.No, 0, P.Mo, P.No, i0, j0,
+        tile_store<T>(sum, (float *)P.ws + (size_t)(slot0 + t) * P.Mo * P.No, P.No, 0, P.Mo, P.No, i0, j0,
                       smem);
     }
 }
@@ -1152,46 +1202,48 @@ __device__ __forceinline__ void group_tile(float *smem, const Prob &P, int local
     }
     const int z = local / P.tiles, tile = local % P.tiles;
     const int i0 = (tile / P.tiles_n) * T::BM, j0 = (tile % P.tiles_n) * T::BN;
-    f32x16 acc[T::FM][T::FN][T::NCH];
+    f32x16 acc[T::FM][T::FN][T::NCH], sum[T::FM][T::FN];
     zero_acc(acc);
     if (P.splits > 1) {
         const Seg &s = P.seg[0];
         const int rbeg = z * P.rps, rend = min(s.R, rbeg + P.rps);
         tile_accumulate<T, LA, LB, true>(smem, s.A, s.B, s.lda, s.ldb, i0, j0, P.Mo, P.No, rbeg, rend, acc);
-        tile_fix<T, false>(acc, i0, j0, P.Mo, P.No, [&](int i, int jt) {
-            return slow_dot<T, LA, LB>(s.A, s.B, s.lda, s.ldb, i, j0, jt, rbeg, rend, 0.f);
+        tile_sum<T>(acc, sum);
+        tile_fix<T>(sum, i0, P.Mo, [&](f32x16 &c, int i, int jt, float scale) {
+            fp32_block<T, LA, LB>(c, lane_base<LA>(s.A, i, s.lda), lane_base<LB>(s.B, min(j0 + jt, P.No - 1), s.ldb),
+                                  s.lda, s.ldb, rbeg, rend, scale);
         });
-        tile_store<T>(acc, (float *)P.ws + (size_t)z * P.Mo * P.No, P.No, 0, P.Mo, P.No, i0, j0, smem);
+        tile_store<T>(sum, (float *)P.ws + (size_t)z * P.Mo * P.No, P.No, 0, P.Mo, P.No, i0, j0, smem);
         return;
     }
     for (int k = 0; k < P.nseg; k++) {
         const Seg &s = P.seg[k];
         tile_accumulate<T, LA, LB, true>(smem, s.A, s.B, s.lda, s.ldb, i0, j0, P.Mo, P.No, 0, s.R, acc);
     }
-    tile_fix<T, false>(acc, i0, j0, P.Mo, P.No, [&](int i, int jt) {
-        float x = 0.f;
+    tile_sum<T>(acc, sum);
+    tile_fix<T>(sum, i0, P.Mo, [&](f32x16 &c, int i, int jt, float scale) {
         for (int k = 0; k < P.nseg; k++) {
             const Seg &s = P.seg[k];
-            x = slow_dot<T, LA, LB>(s.A, s.B, s.lda, s.ldb, i, j0, jt, 0, s.R, x);
+            fp32_block<T, LA, LB>(c, lane_base<LA>(s.A, i, s.lda), lane_base<LB>(s.B, min(j0 + jt, P.No - 1), s.ldb),
+                                  s.lda, s.ldb, 0, s.R, scale);
         }
-        return x;
     });
     if (LA == RC && LB == OC && P.fin) {
         // mm with its residual add: C = R + acc (R in `fin`, C's layout)
         float *C = P.C;
         const float *Rr = P.fin;
         const int ld = P.ldc;
-        tile_epi<T>(acc, P.Mo, P.No, i0, j0, smem, [&](int i, int j) { return Rr[(size_t)i * ld + j]; },
+        tile_epi<T>(sum, P.Mo, P.No, i0, j0, smem, [&](int i, int j) { return Rr[(size_t)i * ld + j]; },
                     [&](int i, int j, float v, float r) { st_out<T>(C + (size_t)i * ld + j, r + v); });
         return;
     }
     if constexpr (LA == RC && LB == RC) {
         if (P.epi == TLG_EPI_ROWDOT) {
-            tile_store_dot<T>(acc, P.C, P.ldc, P.Mo, P.No, i0, j0, P.fin, P.X1, smem);
+            tile_store_dot<T>(sum, P.C, P.ldc, P.Mo, P.No, i0, j0, P.fin, P.X1, smem);
             return;
         }
     }
-    tile_store<T>(acc, P.C, P.ldc, P.beta, P.Mo, P.No, i0, j0, smem);
+    tile_store<T>(sum, P.C, P.ldc, P.beta, P.Mo, P.No, i0, j0, smem);
 }
 
 // Work-item mapping of a grouped launch.  The dispatcher deals workgroup b
