@@ -181,3 +181,55 @@ def test_a_nan_does_not_stall_the_launch(lib, op):
     every = us()
     print(op, "finite", finite, "one NaN", one, "all", every, flush=True)
     assert max(one, every) <= 12 * finite, (finite, one, every)
+
+
+# operand magnitudes from where an unscaled third piece would end (2^-110) down
+# to fp32's subnormals
+TINY = [1e-32, 1e-34, 1e-36, 1e-38, 1e-40]
+
+
+def fp32_of(x):
+    """x to the nearest fp32 and that value in fp64, by integers below 2^-126: a
+    library loaded earlier may have set the CPU to flush subnormals."""
+    sub = np.abs(x) < 2.0 ** -126
+    k = np.rint(np.where(sub, np.ldexp(x, 149), 0)).astype(np.int64)
+    f = np.where(sub, 1.0, x).astype(np.float32)
+    bits = np.where(sub, np.abs(k) | (k < 0).astype(np.int64) << 31, f.view(np.uint32).astype(np.int64))
+    return bits.astype(np.uint32).view(np.float32), np.where(sub, np.ldexp(k.astype(np.float64), -149), f.astype(np.float64))
+
+
+def check_tiny(lib, op, grouped, shape, scale):
+    """One operand at `scale`, the other so large that the sums are ordinary
+    numbers, below 2^112 and past it (where the tiles take the fp32 blocks):
+    the bound of test_error_against_fp64."""
+    M, K, N = shape
+    r = np.random.default_rng(K + N)
+    names = {"mm": ("X", "W"), "mm_bt": ("dY", "W"), "mm_atb": ("X", "dY")}[op]
+    dims = {"X": (M, K), "W": (K, N), "dY": (M, N)}
+    tol = 4 * 2.0 ** -24 * (1 + np.sqrt(reduction(op, M, K, N) / 16))
+    for small, big in (names, names[::-1]):
+        for large in {min(1 / scale, 1e30), min(1 / scale, 1e36)}:
+            o = {n: np.zeros(d, np.float32) for n, d in dims.items()}
+            o64 = {n: np.zeros(d) for n, d in dims.items()}
+            o[small], o64[small] = fp32_of(scale * r.standard_normal(dims[small]))
+            o[big], o64[big] = fp32_of(large * r.standard_normal(dims[big]))
+            ref = want(op, o64["X"], o64["W"], o64["dY"])
+            got = run(lib, op, o["X"], o["W"], o["dY"], grouped)
+            err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+            assert err <= tol, (op, grouped, shape, scale, large, small, err, tol)
+
+
+@pytest.mark.parametrize("scale", TINY)
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_tiny_operands(lib, op, grouped, scale):
+    for shape in ((40, 36, 52), (200, 132, 260)) + (() if grouped else ((67, 61, 254),)):
+        check_tiny(lib, op, grouped, shape, scale)
+
+
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+@pytest.mark.parametrize("pin", PINNED, ids=str)
+def test_tiny_operands_on_every_shape(lib, op, pin):
+    with pinned(lib, *pin):
+        for scale in (1e-36, 1e-40):
+            check_tiny(lib, op, pin[0], (200, 132, 260), scale)

@@ -21,7 +21,7 @@
 // fp32 MFMA chain's, which rounds at every step: 2.5 to 3 times, at 32 to 8192
 // steps (2.9e-7 -> 0.9e-7 at 256, 1.7e-6 -> 5.7e-7 at 8192, N(0, 1) values).
 //
-// What bounds it: matrix cores, vector instructions (11 per pair of values to
+// What bounds it: matrix cores, vector instructions (13 per pair of values to
 // split), LDS (6 bytes per value written, then read by each wave that shares
 // it) and the loads all want more than half of a stage's cycles.  With reads,
 // splits and loads left out the 128x128 tile's MFMAs alone run at 319 TFLOP/s
@@ -66,9 +66,15 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 enum { RC = 0, OC = 1 };
 
-// x = h + m + l in bf16 pieces, each the round to nearest of what the ones
-// before it leave: 3 x 8 significant bits hold an fp32's 24, so the sum is x
-// itself (for |x| below bf16's largest and pieces above its subnormals).
+// 2^16 x = h + m + l in bf16 pieces, each the round to nearest of what the ones
+// before it leave: 3 x 8 significant bits hold an fp32's 24, and bf16's smallest
+// step, 2^-133, is 2^16 times fp32's, so the sum is exact down to fp32's last
+// subnormal (unscaled, l ended at |x| = 2^-110: normwise errors of 2.7e-5 at
+// 1e-36, 2.6e-3 at 1e-38).  tile_sum takes the 2^32 of a product back out.
+// Operands from 2^112 and sums from 2^96 on overflow: tile_fix forms them.  The
+// two multiplications cost 0 to 2 % (8192 x 384 x 2048, forward and backward,
+// 244 -> 248 us; m8 training step 6.90 -> 7.06 ms); m and l alone times 2^16,
+// with a third accumulator for their products, cost the m8 step 7 %.
 // Only plain vector instructions: up to six of them run under each MFMA for
 // nothing (measured: 33 cycles with 0 to 6, + 4 for each further one), where
 // v_dot2c_f32_bf16, which would give a remainder in one instruction, stalls
@@ -80,6 +86,7 @@ __device__ __forceinline__ void split2(float x0, float x1, unsigned &h, unsigned
     asm("" : "+v"(mask));
     auto lo = [](unsigned p) { return __builtin_bit_cast(float, p << 16); };
     auto hi = [&](unsigned p) { return __builtin_bit_cast(float, p & mask); };
+    x0 *= 0x1p16f, x1 *= 0x1p16f;
     h = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
     const float r0 = x0 - lo(h), r1 = x1 - hi(h);
     m = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{r0, r1}), bf16x2));
@@ -481,7 +488,7 @@ __device__ __forceinline__ void tile_accumulate(float *__restrict__ smem, const 
             read(fr[(k + 1) & 1], lds + ((st + 1) & 1) * (SA + SB));
             compute(fr[k & 1]);
             put(la[(k + 2) % NR], lb[(k + 2) % NR], st + 2);
-            sched_step<T, 22 * (LoadA::PER + LoadB::PER) + 8, 3 * (LoadA::PER / LoadA::Ptr::W + LoadB::PER / LoadB::Ptr::W),
+            sched_step<T, 26 * (LoadA::PER + LoadB::PER) + 8, 3 * (LoadA::PER / LoadA::Ptr::W + LoadB::PER / LoadB::Ptr::W),
                        3 * (T::FM * (LA == OC ? 2 : 1) + T::FN * (LB == OC ? 2 : 1))>();
         };
         int st = 0;
@@ -560,11 +567,10 @@ __device__ __forceinline__ void fp32_block(f32x16 &c, const float *__restrict__ 
 }
 
 // Outputs that came out infinite or NaN, again in plain fp32.  An operand that
-// is not finite (or rounds to bf16's infinity) has no split: its pieces turn
-// every sum they enter into NaN where fp32 has infinities, or finite sums of
-// products past the pieces' range.  block(c, i, jt, scale): c += scale^2 times
-// the wave's share of the 32x32 block in which this lane's rows of A and B are
-// row i and tile column jt.  What is still not finite is summed once more at
+// is not finite (or from 2^112 on) has no split: its pieces turn every sum they
+// enter into NaN where fp32 has infinities, or finite sums.  block(c, i, jt,
+// scale): c += scale^2 times the wave's share of the 32x32 block in which this
+// lane's rows of A and B are row i and tile column jt.  What is still not finite is summed once more at
 // 2^-140: the fp32 MFMA rounds a product that is out of range to infinity, and
 // two of them that cancel to NaN.  No wave waits for another here, and finite
 // tiles only look.
@@ -849,14 +855,15 @@ __device__ __forceinline__ void tile_swiglu(const f32x16 (&acc)[T::FM][T::FN], f
     }
 }
 
-// The tile's sums: what the large products' and the small ones' accumulators hold.
+// The tile's sums: what the large products' and the small ones' accumulators hold
+// (of operands times 2^16).
 template <class T>
 __device__ __forceinline__ void tile_sum(const f32x16 (&acc)[T::FM][T::FN][T::NCH], f32x16 (&sum)[T::FM][T::FN])
 {
 #pragma unroll
     for (int a = 0; a < T::FM; a++)
 #pragma unroll
-        for (int b = 0; b < T::FN; b++) sum[a][b] = acc[a][b][0] + acc[a][b][1];
+        for (int b = 0; b < T::FN; b++) sum[a][b] = (acc[a][b][0] + acc[a][b][1]) * 0x1p-32f;
 }
 
 template <int FM, int FN, int NCH>
