@@ -233,3 +233,20 @@ def test_tiny_operands_on_every_shape(lib, op, pin):
     with pinned(lib, *pin):
         for scale in (1e-36, 1e-40):
             check_tiny(lib, op, pin[0], (200, 132, 260), scale)
+
+
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+@pytest.mark.parametrize("R", [1, 2, 3])
+def test_shortest_reductions(lib, op, R):
+    """R steps are R roundings of 2^-24 of the terms' absolute sum, as in fp32, on
+    every tile shape: the piece products that are left out add nothing to it."""
+    M, K, N = {"mm": (300, R, 260), "mm_bt": (300, 260, R), "mm_atb": (R, 300, 260)}[op]
+    r = np.random.default_rng(R)
+    X, W, dY = (r.standard_normal(s, dtype=np.float32) for s in ((M, K), (K, N), (M, N)))
+    bound = R * 2.0 ** -24 * want(op, *(np.abs(t) for t in (X, W, dY)))
+    for pin in PINNED + [(False, -1, 0), (True, -1, 0)]:
+        if pin[0] and op != "mm_atb":
+            continue                       # grouped calls take reductions of whole float4s there
+        with pinned(lib, *pin):
+            err = np.abs(run(lib, op, X, W, dY, pin[0]) - want(op, X, W, dY))
+        assert (err <= bound).all(), (op, R, pin, (err / bound).max())

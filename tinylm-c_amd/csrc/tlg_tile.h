@@ -577,8 +577,12 @@ __device__ __forceinline__ void fp32_block(f32x16 &c, const float *__restrict__ 
 // 8192 x 384 x 2048, fwd / dX / dW us: finite 81 / 99 / 95; one NaN in each
 // operand 200 / 403 / 570, NaN everywhere 410 / 510 / 646 (one lane per output,
 // 1436 / 4839 / 8101 and 5348 / 15192 / 17235).
+//
+// A reduction of one or two `steps` is summed here whatever its sums are: six
+// piece products round a lone product worse than fp32 does (off by up to 9.6e-8
+// of it, 6.0e-8 in fp32; two steps 1.29e-7 and 1.14e-7; from three on better).
 template <class T, class Block>
-__device__ __forceinline__ void tile_fix(f32x16 (&sum)[T::FM][T::FN], int i0, int Mo, Block block)
+__device__ __forceinline__ void tile_fix(f32x16 (&sum)[T::FM][T::FN], int i0, int Mo, int steps, Block block)
 {
     auto finite = [](float x) { return fabsf(x) <= 3.402823466e38f; };
     unsigned need = 0;                                // blocks with a sum that is not finite
@@ -587,7 +591,7 @@ __device__ __forceinline__ void tile_fix(f32x16 (&sum)[T::FM][T::FN], int i0, in
         float z = 0.f;                                // NaN if any is not
 #pragma unroll
         for (int v = 0; v < 16; v++) z = fmaf(sum[n / T::FN][n % T::FN][v], 0.f, z);
-        if (__any(z != z)) need |= 1u << n;
+        if (steps <= 2 || __any(z != z)) need |= 1u << n;
     }
     if (!need) return;
     const int o = threadIdx.x & 31;
@@ -606,7 +610,7 @@ __device__ __forceinline__ void tile_fix(f32x16 (&sum)[T::FM][T::FN], int i0, in
                     auto &x = sum[k / T::FN][k % T::FN];
 #pragma unroll
                     for (int v = 0; v < 16; v++) {
-                        if (!finite(x[v])) x[v] = c[v] * back * back;
+                        if (!finite(x[v]) || (steps <= 2 && back == 1.f)) x[v] = c[v] * back * back;
                         wild |= !finite(x[v]);
                     }
                 }
@@ -907,7 +911,7 @@ __global__ __launch_bounds__(T::THREADS) void k_gemm(GemmArgs g)
     zero_acc(acc);
     tile_accumulate<T, LA, LB, VEC>(smem, g.A, g.B, g.lda, g.ldb, i0, j0, g.Mo, g.No, rbeg, rend, acc);
     tile_sum<T>(acc, sum);
-    tile_fix<T>(sum, i0, g.Mo, [&](f32x16 &c, int i, int jt, float scale) {
+    tile_fix<T>(sum, i0, g.Mo, g.R, [&](f32x16 &c, int i, int jt, float scale) {
         fp32_block<T, LA, LB>(c, lane_base<LA>(g.A, i, g.lda), lane_base<LB>(g.B, min(j0 + jt, g.No - 1), g.ldb),
                               g.lda, g.ldb, rbeg, rend, scale);
     });
@@ -1097,7 +1101,7 @@ __device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int loca
                                   acc);
         }
         tile_sum<T>(acc, sum);
-        tile_fix<T>(sum, i0, rows, [&](f32x16 &c, int i, int jt, float scale) {
+        tile_fix<T>(sum, i0, rows, P.seg[0].R, [&](f32x16 &c, int i, int jt, float scale) {
             // a paired tile's columns alternate between B and B2 (TilePtr PB)
             const bool pair = LA == RC && LB == OC && P.B2;
             constexpr int U = pair_unit(T::BN);
@@ -1166,7 +1170,7 @@ __device__ __forceinline__ void expert_tile(float *smem, const Prob &P, int loca
         // A's reduction rows are sorted rows; gathered ones map through amap
         expert_acc<T, LA, LB>(smem, P, s, s.A, s.B, P.amap, i0, j0, P.Mo, P.No, rbeg, rend, acc);
         tile_sum<T>(acc, sum);
-        tile_fix<T>(sum, i0, P.Mo, [&](f32x16 &c, int i, int jt, float scale) {
+        tile_fix<T>(sum, i0, P.Mo, rows, [&](f32x16 &c, int i, int jt, float scale) {
             const float *pa = lane_base<LA>(s.A, i, s.lda), *pb = lane_base<LB>(s.B, min(j0 + jt, P.No - 1), s.ldb);
             if (P.amap) fp32_block<T, LA, LB, true>(c, pa, pb, s.lda, s.ldb, rbeg, rend, scale, P.amap);
             else        fp32_block<T, LA, LB>(c, pa, pb, s.lda, s.ldb, rbeg, rend, scale);
@@ -1216,7 +1220,7 @@ __device__ __forceinline__ void group_tile(float *smem, const Prob &P, int local
         const int rbeg = z * P.rps, rend = min(s.R, rbeg + P.rps);
         tile_accumulate<T, LA, LB, true>(smem, s.A, s.B, s.lda, s.ldb, i0, j0, P.Mo, P.No, rbeg, rend, acc);
         tile_sum<T>(acc, sum);
-        tile_fix<T>(sum, i0, P.Mo, [&](f32x16 &c, int i, int jt, float scale) {
+        tile_fix<T>(sum, i0, P.Mo, s.R, [&](f32x16 &c, int i, int jt, float scale) {
             fp32_block<T, LA, LB>(c, lane_base<LA>(s.A, i, s.lda), lane_base<LB>(s.B, min(j0 + jt, P.No - 1), s.ldb),
                                   s.lda, s.ldb, rbeg, rend, scale);
         });
@@ -1228,7 +1232,7 @@ __device__ __forceinline__ void group_tile(float *smem, const Prob &P, int local
         tile_accumulate<T, LA, LB, true>(smem, s.A, s.B, s.lda, s.ldb, i0, j0, P.Mo, P.No, 0, s.R, acc);
     }
     tile_sum<T>(acc, sum);
-    tile_fix<T>(sum, i0, P.Mo, [&](f32x16 &c, int i, int jt, float scale) {
+    tile_fix<T>(sum, i0, P.Mo, P.seg[0].R, [&](f32x16 &c, int i, int jt, float scale) {
         for (int k = 0; k < P.nseg; k++) {
             const Seg &s = P.seg[k];
             fp32_block<T, LA, LB>(c, lane_base<LA>(s.A, i, s.lda), lane_base<LB>(s.B, min(j0 + jt, P.No - 1), s.ldb),
