@@ -66,7 +66,14 @@ void *tlg_mirror(const void *host);
 /* ---- device pointers, asynchronous on `stream` -------------------------- */
 /* Same arithmetic as the drop-in entries on device-resident buffers; returns
  * TLG_OK once the kernels are enqueued.  These are what a device-resident
- * caller (the step drivers in tinylm-c_amd/host) uses. */
+ * caller (the step drivers in tinylm-c_amd/host) uses.
+ * Streams: outputs of at least 240 tiles of 64 x 64 are formed whole, and such
+ * calls may overlap on different streams.  A smaller output (and any with at
+ * most 8 rows) may split a long reduction over workgroups, whose partial sums
+ * lie in the library's one workspace: those calls must not overlap.
+ * Operands may hold any fp32 value, subnormals included; where infinities, NaN
+ * or magnitudes from 2^112 on (sums from 2^96 on) are met, the tiles they enter
+ * take 2 to 8 times as long. */
 int tlg_dev_sgemm_nn(float *Y, const float *X, const float *W, int M, int K, int N, void *stream);
 int tlg_dev_sgemm_nt_acc(float *dX, const float *dY, const float *W, int M, int K, int N, void *stream);
 int tlg_dev_sgemm_tn_acc(float *dW, const float *X, const float *dY, int M, int K, int N, void *stream);

@@ -250,3 +250,26 @@ def test_shortest_reductions(lib, op, R):
         with pinned(lib, *pin):
             err = np.abs(run(lib, op, X, W, dY, pin[0]) - want(op, X, W, dY))
         assert (err <= bound).all(), (op, R, pin, (err / bound).max())
+
+
+@pytest.mark.parametrize("call", [("mm", 4096, 2048, 384), ("mm_bt", 4096, 384, 2048), ("mm_atb", 8192, 1024, 1024),
+                                  ("mm", 1024, 4096, 960)], ids=str)
+def test_large_outputs_run_whole(lib, call):
+    """From 240 64x64 tiles on no call splits its reduction: a split's partials
+    lie in a workspace that a call on another stream would write too."""
+    assert lib.kernel_name(*call)[1] == 1
+    torch = _torch()
+    op, M, K, N = call
+    dims = {"mm": ((M, K), (K, N), (M, N)), "mm_bt": ((M, N), (K, N), (M, K)), "mm_atb": ((M, K), (M, N), (K, N))}[op]
+    f = {"mm": lib.mm, "mm_bt": lib.mm_bt, "mm_atb": lib.mm_atb}[op]
+    torch.manual_seed(1)
+    one, two, both = [], [], [torch.cuda.Stream() for _ in range(2)]
+    ops = [tuple(torch.randn(*s, device="cuda") for s in dims[:2]) for _ in both]
+    for outs, streams in ((one, both[:1] * 2), (two, both)):
+        outs += [torch.zeros(*dims[2], device="cuda") for _ in both]
+        torch.cuda.synchronize()
+        for _ in range(4):
+            for (a, b), c, s in zip(ops, outs, streams):
+                f(c.data_ptr(), a.data_ptr(), b.data_ptr(), M, K, N, s.cuda_stream)
+        torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(one, two))

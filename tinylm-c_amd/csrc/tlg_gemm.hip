@@ -55,6 +55,7 @@ static int tile_name(const TileCfg &c, char *buf, int len)
 static inline bool al16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
+#define TLG_WHOLE_TILES 240           // 64x64 tiles of an output whose reduction is never split
 struct GemmPlan { int ci; int tiles_n, tiles, splits, rps; };
 
 // Forced choice for tuning sweeps (tlg_tune_force); -1 = automatic.
@@ -90,12 +91,17 @@ static GemmPlan make_plan(int ci, int Mo, int No, int R, int splits, size_t ws_f
 // 64-step stages (8 waves, a quarter of each stage per wave) from 512 steps
 // on and 16-step stages below: 14.5 against 16.8 us at 768 steps, 7.5 against
 // 8.0 at 128.
+//
+// Outputs of 240 64x64 tiles and more run whole: a split's partials lie in the
+// one workspace, which calls that overlap on two streams would both write, and
+// outputs of that size are promised not to (@MEASURED@).
 static GemmPlan plan_gemm(int Mo, int No, int R, size_t ws_floats)
 {
     if (g_force_cfg >= 0 && g_force_cfg < kNumCfgs)
         return make_plan(g_force_cfg, Mo, No, R, g_force_splits, ws_floats);
     const int enough = 160;
     const int order[] = {9, R >= 512 ? 8 : 3, 15};
+    const bool whole = (long long)cdiv(Mo, 64) * cdiv(No, 64) >= TLG_WHOLE_TILES;
     int ci = 15, splits = 1;
     for (int k = 0; k < 3; k++) {
         const TileCfg &c = kCfgs[order[k]];
@@ -104,6 +110,7 @@ static GemmPlan plan_gemm(int Mo, int No, int R, size_t ws_floats)
         splits = tiles >= enough ? 1 : cdiv(enough, (int)tiles);
         const int maxs = R / (k == 2 ? 256 : 512);
         if (splits > maxs) splits = maxs > 1 ? maxs : 1;
+        if (whole) splits = 1;
         if (tiles * splits >= enough) break;
     }
     return make_plan(ci, Mo, No, R, splits, ws_floats);
