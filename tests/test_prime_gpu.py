@@ -80,3 +80,20 @@ def test_prime_refuses_what_chunks_refuse(lib):
     d.prime(np.full(48, 5, np.int32), s)
     assert d.state(s)[0] == 48
     lib.tlg_stream_destroy(s)
+
+
+def test_a_bad_token_past_the_ring_starts_nothing(lib):
+    """Refused before any row of the prompt is copied or run: the rings stay."""
+    import tlgemm
+    s = lib.tlg_stream_create()
+    d = tlgemm.host().decode(KW, 32, kv_f16=0, exact_exp=1, maxpos=128, mmax=8, pool=1)
+    d.upload(StepFns("oracle").init_params(model(**KW), 3), s)
+    d.prime(np.full(40, 5, np.int32), s)
+    rings = [d.ring(l, s) for l in range(KW["L"])]
+    bad = np.full(100, 7, np.int32)
+    bad[90] = KW["V"]
+    with pytest.raises(tlgemm.TlgError):
+        d.prime(bad, s)
+    for l, ring in enumerate(rings):
+        assert all(np.array_equal(x, y) for x, y in zip(ring, d.ring(l, s)))
+    lib.tlg_stream_destroy(s)

@@ -462,18 +462,22 @@ int tl_decode_chunk(TlDecode *d, const int *tok, int m, int start, void *st)
 
 /* A prompt's rows through run_bulk: all of them when they fit the ring, else
  * the whole chunks of mmax rows that lie below W; *done = the rows taken,
- * *last = the last chunk's rows if it is among them. */
+ * *last = the last chunk's rows if it is among them.  Every token is looked at
+ * before the first copy from the caller's prompt is enqueued, so no later
+ * chunk refuses one with that copy still in flight.
+ * From two chunks' rows ahead of the last one on: 25 tokens take 0.47 ms in one
+ * pass and 1.70 in chunks (m8 model, mmax 8).  The pass already wins at 9 (0.46
+ * against 0.73 ms; nano 79 against 185 us), where the chunks still run. */
 static int prime_bulk(TlDecode *d, const int *prompt, int n, int *done, int *last, void *st)
 {
     const int tail = (n - 1) % d->mmax + 1;
     const int rows = n <= d->W ? n : d->W / d->mmax * d->mmax;
     *done = 0;
     if (d->unfused || !d->bulk || rows - tail < 2 * TLD_MAXM || n > d->maxpos) return 0;
-    for (int j = 0; j < rows; j++) if (prompt[j] < 0 || prompt[j] >= d->m.V) return TLG_EINVAL;
+    for (int j = 0; j < n; j++) if (prompt[j] < 0 || prompt[j] >= d->m.V) return TLG_EINVAL;
+    /* pieces before the last are whole chunks (bulk is), so none cuts the tail */
     for (int i = 0, m; i < rows; i += m) {
         m = rows - i < d->bulk ? rows - i : d->bulk;
-        /* the tail in one piece */
-        if (rows == n && i + m < n && i + m > n - tail) m = n - tail - i;
         CK(run_bulk(d, prompt + i, m, i, rows == n && i + m == n ? tail : 0, st));
     }
     *done = rows;
@@ -518,7 +522,7 @@ int tl_decode_generate_spec(TlDecode *d, const int *prompt, int np, int n, int *
 {
     const int K = d ? d->m.n_mtp : 0;
     if (!d || !prompt || np <= 0 || n <= 0 || !toks || K < 1 || K + 1 > d->mmax || K + 1 > 16) return TLG_EINVAL;
-    /* prefill in chunks of mmax (positions 0..np-1), as tl_decode_prime */
+    /* prefill of positions 0..np-1, as tl_decode_prime */
     int i = 0, m = 0;
     CK(prime_bulk(d, prompt, np, &i, &m, st));
     while (i < np) {
