@@ -173,10 +173,13 @@ int tlg_gemv_status(void);
  * the kernel's tile table; -1 = automatic: the largest of 128x128, 128x64,
  * 64x64, 64x32 and 32x32 tiles that gives a launch enough work items). */
 int tlg_tune_group(int cfg);
-/* Tuning hook: a policy in place of the automatic one -- candidate tile configs
- * (up to 3, first that yields min_waves x 256 work items wins, else the last; ncands
- * 0 keeps the list), min_waves (<= 0 keeps it) and the target reduction
- * steps per split work item (0 keeps it).  Applies to later launches. */
+/* Tuning hook: the automatic policy.  cands: tile configs in place of its own
+ * list (up to 3, the first that yields min_waves x 256 work items wins, else
+ * the last; ncands 0 keeps what is set, one candidate of -1 puts the automatic
+ * list back).  min_waves (0 keeps it, 3 at the start): the automatic list's
+ * thresholds, the expert launches' too, count min_waves / 3 times.  rtarget:
+ * the target reduction steps per split work item (0 keeps it).  Applies to
+ * later launches. */
 int tlg_tune_group_policy(const int *cands, int ncands, double min_waves, int rtarget);
 /* Tuning hook: pin the target reduction steps per work item of the split
  * (mm_atb) problems of later grouped launches: >= 64 splits every long

@@ -3,6 +3,7 @@ products of them on the matrix cores.  Error against fp64, operands that have
 no such split (infinities, NaN, magnitudes past bf16's largest), and the
 sizes where a tile, a stage or a chunk ends."""
 import contextlib
+import ctypes
 
 import numpy as np
 import pytest
@@ -273,3 +274,32 @@ def test_large_outputs_run_whole(lib, call):
                 f(c.data_ptr(), a.data_ptr(), b.data_ptr(), M, K, N, s.cuda_stream)
         torch.cuda.synchronize()
     assert all(torch.equal(x, y) for x, y in zip(one, two))
+
+
+def test_tile_policy_hook(lib):
+    """A list of candidates takes the automatic one's place and a candidate of -1
+    puts it back; min_waves scales whichever is there."""
+    torch = _torch()
+    M, K, N = 4096, 256, 768
+    x, w, y = (torch.randn(*s, device="cuda") for s in ((M, K), (K, N), (M, N)))
+
+    def shape():
+        lib.group([dict(op="mm", C=y.data_ptr(), M=M, K=K, N=N, A=[x.data_ptr()], B=[w.data_ptr()])])
+        torch.cuda.synchronize()
+        return lib.tlg_group_kernel().decode()
+
+    def policy(cands, min_waves=0.0):
+        c = (ctypes.c_int * max(1, len(cands)))(*cands)
+        return lib.tlg_tune_group_policy(c, len(cands), min_waves, 0)
+
+    start = shape()
+    try:
+        assert policy([], 30.0) == 0 and "Tile<64, 32, " in shape() and "Tile<64, 32, " not in start
+        assert policy([], 3.0) == 0 and shape() == start
+        assert policy([33, 15]) == 0 and "Tile<32, 32, " in shape()          # 192 of 768 items
+        assert policy([], 0.5) == 0 and "Tile<128, 128, " in shape()
+        assert policy([-1], 3.0) == 0 and shape() == start
+        for bad in ([2], [99], [-1, 3], [-2]):
+            assert policy(bad) != 0 and shape() == start
+    finally:
+        lib.check(policy([-1], 3.0), "policy")

@@ -305,9 +305,10 @@ static int flush_foreign(hipStream_t st);
 //   64x64 of 8 waves, each 64x32 of a quarter of a 64-step stage: one item per
 //            CU, so the waves come from the reduction (m3 W2 16.1 / 18.8)
 //   64x32, 32x32 likewise (nano head backward 23 / 28 / 29, W2 7.0 on 32x32)
-// mm_atb splits aim for about 512 reduction steps.  TLG_GROUP_CANDS,
-// TLG_GROUP_MINWAVES and TLG_GROUP_RTARGET (or tlg_tune_group_policy) put a
-// list of their own in its place, tlg_tune_group pins one shape.
+// mm_atb splits aim for about 512 reduction steps.  TLG_GROUP_CANDS (or
+// tlg_tune_group_policy) puts a list of its own in the rows' place,
+// TLG_GROUP_MINWAVES scales the rows' items (3 = as they stand), tlg_tune_group
+// pins one shape.
 static const struct { int cfg, items; } kAuto[] = {{33, 160}, {34, 240}, {35, 320}, {41, 160}, {21, 128}, {15, 0}};
 static int g_group_cfg = -1;
 static int g_group_rt = 0;               // split target pinned for the next launches (tlg_tune_group_split)
@@ -381,7 +382,8 @@ extern "C" int tlg_tune_group_policy(const int *cands, int ncands, double min_wa
     group_env();
     if (ncands < 0 || ncands > 3 || (ncands > 0 && !cands) || min_waves < 0 || (rtarget && rtarget < 64))
         return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: bad arguments");
-    for (int k = 0; k < ncands; k++)
+    const bool automatic = ncands == 1 && cands[0] == -1;
+    for (int k = 0; k < ncands && !automatic; k++)
         if (cands[k] < 0 || cands[k] >= kNumCfgs || cands[k] == 2 || (cands[k] >= 5 && cands[k] <= 7))
             return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: config %d", cands[k]);
     if (ncands > 0) {
@@ -720,7 +722,7 @@ int tlg_group_launch(const TlgGemmCall *calls, int n, hipStream_t st)
         for (const auto &row : kAuto) {
             ci = row.cfg;
             const double items = items_of(ci);
-            if (items < row.items) continue;
+            if (items < row.items * (g_min_waves / 3.0)) continue;
             if (ci == 33 && !tn) {
                 const double rounds = items / 256.0;
                 if (rounds < (rounds > 1.0 ? 1.7 : 0.7)) continue;
@@ -1016,10 +1018,11 @@ int tlg_expert_launch(const TlgExpertCall *calls, int n, const int *eoff, int E,
         }
         return t;
     };
+    const double by = g_min_waves / 3.0;
     const int ci = g_expert_cfg >= 0 ? g_expert_cfg
-                 : items_for(expert_shape(9)) >= 160 ? 9
-                 : items_for(expert_shape(3)) >= 320 ? 3
-                 : items_for(expert_shape(14)) >= 320 ? 14 : 15;
+                 : items_for(expert_shape(9)) >= 160 * by ? 9
+                 : items_for(expert_shape(3)) >= 320 * by ? 3
+                 : items_for(expert_shape(14)) >= 320 * by ? 14 : 15;
     const TileCfg tc = expert_shape(ci);
     GroupArgs a, red, pend;
     a.nprob = red.nprob = pend.nprob = 0;
