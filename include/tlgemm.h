@@ -189,11 +189,11 @@ int tlg_tune_group_policy(const int *cands, int ncands, double min_waves, int rt
 int tlg_tune_group_split(int rtarget);
 /* Tuning hook: the tile shape of the MoE expert launches (tlg_dev_moe_*):
  * cfg -1 = automatic (128x128 tiles when a launch has about 160 of them, else
- * 64x64, 64x32 or 32x32), or 3 (64x64), 18 (64x64, wave pairs
+ * 64x64, 64x32 or 32x32), or 9 (128x128), 3 (64x64), 18 (64x64, wave pairs
  * each taking half of a 32-step stage), 14 (64x32), 15 (32x32), 22 (8-wave
  * 64x64, whose waves split each 64-step stage four ways) pinned;
- * sched 0 or 1 = plain stores, 2 = streaming stores, -1 = automatic (2 for the fused SwiGLU launches of dense rows, 1 for
- * MoE launches).  Applies to later launches. */
+ * sched 0 or 1 = plain stores, 2 = streaming stores, -1 = automatic (2 for the
+ * fused SwiGLU launches of dense rows, 1 for MoE launches).  Applies to later launches. */
 int tlg_tune_expert(int cfg, int sched);
 
 /* ---- top-1 mixture-of-experts FFN --------------------------------------- */

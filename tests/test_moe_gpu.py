@@ -256,7 +256,23 @@ def test_expert_tile_forms(lib, orc, cfg, sched):
     assert lib.tlg_tune_expert(8, 1) != 0 and lib.tlg_tune_expert(3, 3) != 0
 
 
-@pytest.mark.parametrize("cfg", [-1, 3, 14, 15, 18, 22])
+@pytest.mark.parametrize("cfg", [9, 3, 14, 15, 18, 22])
+@pytest.mark.parametrize("sched", [1, 2])
+@pytest.mark.parametrize("dims", [(4096, 256, 768, 4, 2.0), (263, 132, 196, 2, 0.0), (521, 260, 100, 4, 0.0),
+                                  (300, 36, 324, 2, 0.0)], ids=str)
+def test_every_expert_shape_ragged(lib, orc, cfg, sched, dims):
+    """Each shape of the expert launches at row counts just past 128 and at widths
+    that leave a part of a 64- or 128-wide column tile, of a pair's 32 columns and
+    of a stage."""
+    N, D, F, E, skew = dims
+    lib.check(lib.tlg_tune_expert(cfg, sched), "tune expert")
+    try:
+        test_against_oracle_and_f64(lib, orc, N, D, F, E, skew, ())
+    finally:
+        lib.check(lib.tlg_tune_expert(-1, -1), "tune expert")
+
+
+@pytest.mark.parametrize("cfg", [-1, 9, 3, 14, 15, 18, 22])
 @pytest.mark.parametrize("dims", [(300, 132, 196, 3), (67, 32, 48, 3)], ids=str)
 def test_operands_without_a_split(lib, cfg, dims):
     """Infinities, NaN and a weight that rounds to bf16's infinity in the expert

@@ -316,13 +316,21 @@ static double g_min_waves = 3.0;
 static int g_cand[4] = {-1, -1, -1, -1};  // candidates put in place of kAuto
 static int g_rtarget = 512;
 static int g_erps = 1024;                // expert TN slice (TLG_EXPERT_RPS)
-static int g_expert_cfg = -1;            // expert tile shape pinned (TLG_EXPERT_CFG: 3, 14, 15, 18, 22)
+static int g_expert_cfg = -1;            // expert tile shape pinned (TLG_EXPERT_CFG: a key of TLG_EXPERTS)
 static int g_expert_sched = -1;          // expert tiles: 0, 1 plain stores, 2 streaming ones, -1 automatic: 2 for launches of
                                          // dense rows (the training step's fused SwiGLU: 2.003 -> 1.995 ms), 1 for
                                          // MoE launches (streaming measured 0.232 -> 0.237 ms per kept pair: the
                                          // next launch reads their g, u, a, y right away) (TLG_EXPERT_SCHED)
 static int g_group_last = 3;          // shape of the most recent grouped launch
 static const char *g_group_last_name = nullptr;   // set when that launch was a GEMV group
+
+static bool is_expert_shape(int key)
+{
+#define TLG_ROW(k, bm, bn, bk, wgm, wk, nw) if (key == k) return true;
+    TLG_EXPERTS(TLG_ROW)
+#undef TLG_ROW
+    return false;
+}
 
 static void group_env(void)
 {
@@ -346,7 +354,7 @@ static void group_env(void)
     e = getenv("TLG_EXPERT_RPS");
     if (e && atoi(e) >= 64) g_erps = atoi(e);
     e = getenv("TLG_EXPERT_CFG");
-    if (e && (atoi(e) == 3 || atoi(e) == 14 || atoi(e) == 15 || atoi(e) == 18 || atoi(e) == 22))
+    if (e && is_expert_shape(atoi(e)))
         g_expert_cfg = atoi(e);
     if ((e = getenv("TLG_EXPERT_SCHED")) && atoi(e) >= -1 && atoi(e) <= 2) g_expert_sched = atoi(e);
     e = getenv("TLG_GROUP_RTARGET");
@@ -398,7 +406,7 @@ extern "C" int tlg_tune_group_policy(const int *cands, int ncands, double min_wa
 extern "C" int tlg_tune_expert(int cfg, int sched)
 {
     group_env();
-    if ((cfg != -1 && cfg != 3 && cfg != 14 && cfg != 15 && cfg != 18 && cfg != 22) || sched < -1 || sched > 2)
+    if ((cfg != -1 && !is_expert_shape(cfg)) || sched < -1 || sched > 2)
         return tlg_fail(TLG_EINVAL, "tlg_tune_expert: config %d, order %d", cfg, sched);
     g_expert_cfg = cfg;
     g_expert_sched = sched;
