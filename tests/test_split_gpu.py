@@ -54,7 +54,8 @@ def reduction(op, M, K, N):
     return {"mm": K, "mm_bt": N, "mm_atb": M}[op]
 
 
-# (M, K, N): a tile, stage or chunk ends one short, exactly, or one past
+# (M, K, N): a tile, stage or chunk (of the 32x32 shape; the others' lie among
+# multiples of these) ends one short, exactly, or one past
 EDGES = [(9, 16, 16), (70, 1, 33), (70, 33, 1), (70, 3, 2), (1030, 2, 5), (9, 130, 3), (67, 261, 254), (32, 32, 32), (33, 20, 68), (64, 15, 64), (65, 17, 63), (127, 48, 129), (128, 128, 128),
          (257, 131, 259), (300, 64, 36), (513, 4, 72), (1024, 512, 192), (2050, 72, 516)]
 
@@ -62,6 +63,13 @@ EDGES = [(9, 16, 16), (70, 1, 33), (70, 33, 1), (70, 3, 2), (1030, 2, 5), (9, 13
 @pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
 @pytest.mark.parametrize("shape", EDGES, ids=str)
 def test_error_against_fp64(lib, op, shape):
+    """check_error by the automatic rules (32x32 tiles at all but the largest of
+    these sizes)."""
+    for grouped in (False, True):
+        check_error(lib, op, grouped, shape)
+
+
+def check_error(lib, op, grouped, shape):
     """Each product is exact to 2^-25 and each 16-step MFMA adds one rounding
     of the running sum (2^-24): over R steps the error's 2-norm stays under
     2^-24 (1 + sqrt(R / 16)) times the result's for random signs, with room
@@ -74,12 +82,11 @@ def test_error_against_fp64(lib, op, shape):
     ref = want(op, X, W, dY)
     R = reduction(op, M, K, N)
     tol = 4 * 2.0 ** -24 * (1 + np.sqrt(R / 16))
-    for grouped in (False, True):
-        if grouped and (M % 4 and op == "mm_atb" or K % 4 or N % 4):
-            continue
-        got = run(lib, op, X, W, dY, grouped)
-        err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
-        assert err <= tol, (op, shape, grouped, err, tol)
+    if grouped and (M % 4 and op == "mm_atb" or K % 4 or N % 4):
+        return
+    got = run(lib, op, X, W, dY, grouped)
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert err <= tol, (op, shape, grouped, err, tol)
 
 
 @pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
@@ -131,6 +138,11 @@ def test_magnitudes(lib, scale):
 PINNED = [(False, c, sp) for c in (9, 8, 3, 15) for sp in (1, 3)] + [(True, c, 0) for c in (33, 47, 34, 35, 41, 21, 15)]
 
 
+# extents one short of, at and one past 128 and 256, aligned and odd
+WIDE = [(127, 129, 255), (129, 255, 127), (255, 127, 129), (257, 193, 131), (128, 128, 256), (132, 260, 124),
+        (252, 68, 388), (36, 512, 132), (516, 132, 36)]
+
+
 @contextlib.contextmanager
 def pinned(lib, grouped, cfg, splits):
     lib.check(lib.tlg_tune_group(cfg) if grouped else lib.tlg_tune_force(cfg, splits), "pin")
@@ -138,6 +150,17 @@ def pinned(lib, grouped, cfg, splits):
         yield
     finally:
         lib.check(lib.tlg_tune_group(-1) if grouped else lib.tlg_tune_force(-1, 0), "unpin")
+
+
+@pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
+@pytest.mark.parametrize("pin", PINNED, ids=str)
+def test_error_on_every_shape(lib, op, pin):
+    """The bound of the automatic choice on each tile shape, where the large
+    tiles' rows, columns, stages and chunks end; single calls with rows that are
+    no whole float4s too."""
+    for shape in EDGES + WIDE:
+        with pinned(lib, *pin):
+            check_error(lib, op, pin[0], shape)
 
 
 @pytest.mark.parametrize("op", ["mm", "mm_bt", "mm_atb"])
