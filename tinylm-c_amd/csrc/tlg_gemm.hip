@@ -168,7 +168,7 @@ static int launch_reduce(const float *ws, float *C, int Mo, int No, int ldc, int
 
 // One GEMM on `st` whose split partials (if any) go to ws[0, ws_floats).
 // Allocates nothing: the caller owns ws (the library's workspace, or the
-// no-allocation scratch below).  max_splits caps the reduction split.
+// no-allocation scratch below).
 static int gemm_launch_ws(TlgKind kind, const float *A, const float *B, float *C, int Mo, int No, int R,
                           int lda, int ldb, int ldc, int beta, float *ws, size_t ws_floats, hipStream_t st)
 {
@@ -195,7 +195,8 @@ static int gemm_launch_ws(TlgKind kind, const float *A, const float *B, float *C
     a.splits = pl.splits; a.rps = pl.rps;
     a.ws = ws;
     const int grid = pl.tiles * pl.splits;
-    if (!tlg_single_part0(pl.ci, kind, vec, a, grid, st) && !tlg_single_part1(pl.ci, kind, vec, a, grid, st))
+    const int ci = tile_canon(pl.ci);
+    if (!tlg_single_part0(ci, kind, vec, a, grid, st) && !tlg_single_part1(ci, kind, vec, a, grid, st))
         return tlg_fail(TLG_EINVAL, "GEMM: no kernel for tile configuration %d", pl.ci);
     TLG_HIP(hipGetLastError());
     if (pl.splits > 1) return launch_reduce(ws, C, Mo, No, ldc, pl.splits, beta, st);
@@ -324,6 +325,8 @@ static int g_expert_sched = -1;          // expert tiles: 0, 1 plain stores, 2 s
 static int g_group_last = 3;          // shape of the most recent grouped launch
 static const char *g_group_last_name = nullptr;   // set when that launch was a GEMV group
 
+static bool is_group_shape(int cfg) { return cfg >= 0 && cfg < kNumCfgs && tile_grouped(cfg); }
+
 static bool is_expert_shape(int key)
 {
 #define TLG_ROW(k, bm, bn, bk, wgm, wk, nw) if (key == k) return true;
@@ -340,12 +343,12 @@ static void group_env(void)
     const char *e = getenv("TLG_GROUP_MINWAVES");
     if (e && atof(e) > 0) g_min_waves = atof(e);
     e = getenv("TLG_GROUP_CFG");
-    if (e && *e) g_group_cfg = atoi(e);
+    if (e && *e && is_group_shape(atoi(e))) g_group_cfg = atoi(e);
     e = getenv("TLG_GROUP_CANDS");            // e.g. "3,13,15"
     if (e && *e) {
         int k = 0;
         for (const char *q = e; *q && k < 3; ) {
-            g_cand[k++] = atoi(q);
+            if (is_group_shape(atoi(q))) g_cand[k++] = atoi(q);
             while (*q && *q != ',') q++;
             if (*q == ',') q++;
         }
@@ -376,9 +379,9 @@ static const GroupArgs &group_seal(const GroupArgs &a)
 
 static void launch_group(int ci, const GroupArgs &a, int grid, hipStream_t st)
 {
-    if (ci < 0 || ci >= kNumCfgs) ci = 3;
     const GroupArgs &b = group_seal(a);
-#define TLG_TRY(k) if (!tlg_group_part##k(ci, b, grid, st))
+    const int kernel = tile_canon(ci);
+#define TLG_TRY(k) if (!tlg_group_part##k(kernel, b, grid, st))
     TLG_TILE_PARTS(TLG_TRY) {}
 #undef TLG_TRY
     g_group_last = ci;
@@ -392,7 +395,7 @@ extern "C" int tlg_tune_group_policy(const int *cands, int ncands, double min_wa
         return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: bad arguments");
     const bool automatic = ncands == 1 && cands[0] == -1;
     for (int k = 0; k < ncands && !automatic; k++)
-        if (cands[k] < 0 || cands[k] >= kNumCfgs || cands[k] == 2 || (cands[k] >= 5 && cands[k] <= 7))
+        if (!is_group_shape(cands[k]))
             return tlg_fail(TLG_EINVAL, "tlg_tune_group_policy: config %d", cands[k]);
     if (ncands > 0) {
         for (int k = 0; k < ncands; k++) g_cand[k] = cands[k];
@@ -415,7 +418,7 @@ extern "C" int tlg_tune_expert(int cfg, int sched)
 
 extern "C" int tlg_tune_group(int cfg)
 {
-    if (cfg != -1 && cfg != 0 && cfg != 1 && cfg != 3 && cfg != 4 && (cfg < 8 || cfg >= kNumCfgs))
+    if (cfg != -1 && !is_group_shape(cfg))
         return tlg_fail(TLG_EINVAL, "tlg_tune_group: config %d", cfg);
     g_group_cfg = cfg;
     return TLG_OK;
@@ -743,9 +746,8 @@ int tlg_group_launch(const TlgGemmCall *calls, int n, hipStream_t st)
     }
     // the block-dot epilogue stages a whole tile in the stage buffers: not on
     // the 128 x 128 shapes, whose tile is larger than their stages
-    if (rowdot && ci >= 0 && ci < kNumCfgs && kCfgs[ci].bm * kCfgs[ci].bn > 64 * 128) ci = 38;
-    // geometry of the chosen shape (the sweep variants 9-12 are 64x64 tiles)
-    const TileCfg &tc = kCfgs[(ci >= 0 && ci < kNumCfgs) ? ci : 3];
+    if (rowdot && kCfgs[ci].bm * kCfgs[ci].bn > 64 * 128) ci = 38;
+    const TileCfg &tc = kCfgs[ci];
 
     GroupArgs a;
     a.nprob = 0;

@@ -11,7 +11,7 @@
 template <int I, class T>
 static bool launch_row(int ci, const GroupArgs &a, int grid, hipStream_t st)
 {
-    if constexpr (I % TLG_GROUP_PARTS == TLG_PART) {
+    if constexpr (I % TLG_GROUP_PARTS == TLG_PART && tile_canon(I) == I && tile_grouped(I)) {
         if (ci == I) {
             hipLaunchKernelGGL((k_group<T>), dim3(grid), dim3(T::THREADS), 0, st, a);
             return true;
@@ -39,7 +39,7 @@ static void launch_t(const GemmArgs &a, int grid, bool vec, hipStream_t st)
 template <int I, class T>
 static bool launch_row(int ci, TlgKind kind, bool vec, const GemmArgs &a, int grid, hipStream_t st)
 {
-    if constexpr (I < TLG_SINGLE && I % 2 == TLG_SPART) {
+    if constexpr (I < TLG_SINGLE && I % 2 == TLG_SPART && tile_canon(I) == I) {
         if (ci == I) {
             if (kind == TLG_NN)      launch_t<T, RC, OC>(a, grid, vec, st);
             else if (kind == TLG_NT) launch_t<T, RC, RC>(a, grid, vec, st);
