@@ -421,8 +421,9 @@ def bench_moe(lib, stream, steps):
 
 def probes(lib, stream):
     """Achievable peaks on this box: a streaming copy (k_copy, 1 GiB each
-    way), a streaming read (k_read, 1 GiB) and register-only fp32 MFMA
-    (k_mfma_peak)."""
+    way), a streaming read (k_read, 1 GiB) and register-only MFMA, fp32 and
+    bf16 (k_mfma_peak, k_mfma_bf16_peak; a sixth of the latter is what the
+    tiles' six piece products could reach)."""
     n = 1 << 28
     src, dst = lib.tlg_dev_malloc(4 * n), lib.tlg_dev_malloc(4 * n)
     check(lib.tlg_dev_fill_normal(src, n, 3, 1.0, stream), "fill")
@@ -438,10 +439,14 @@ def probes(lib, stream):
     check(lib.tlg_dev_mfma_peak(dst, blocks, iters, stream), "mfma")
     ms2, _ = time_steps(lib, lambda: lib.tlg_dev_mfma_peak(dst, blocks, iters, stream), stream, 5)
     mfma = blocks * 4 * 4 * iters * 4096.0 / (ms2 / 5 * 1e-3) / 1e12
+    check(lib.tlg_dev_mfma_bf16_peak(dst, blocks, iters, stream), "mfma")
+    ms3, _ = time_steps(lib, lambda: lib.tlg_dev_mfma_bf16_peak(dst, blocks, iters, stream), stream, 5)
+    mfma16 = blocks * 4 * 4 * iters * 32768.0 / (ms3 / 5 * 1e-3) / 1e12
     lib.tlg_dev_free(src)
     lib.tlg_dev_free(dst)
     return {"hbm_copy_gbs": round(hbm, 1), "hbm_read_gbs": round(hbm_read, 1), "copy_bytes_each_way": 4 * n,
-            "mfma_fp32_tflops": round(mfma, 1)}
+            "mfma_fp32_tflops": round(mfma, 1), "mfma_bf16_tflops": round(mfma16, 1),
+            "mfma_bf16_sixth_tflops": round(mfma16 / 6, 1)}
 
 
 def host_cpu_share():
@@ -995,7 +1000,7 @@ def main():
             "kernel": dom_name, "bound": bound, "achieved": round(achieved, 2), "peak": peak,
             "unit": unit, "frac": round(achieved / peak, 4),
             "traffic": read_traffic(dom_name),
-            "frac_of_achievable": round(achieved / peaks[("mfma_fp32_tflops" if bound == "mfma" else "hbm_copy_gbs")], 4)
+            "frac_of_achievable": round(achieved / peaks[("mfma_bf16_sixth_tflops" if bound == "mfma" else "hbm_copy_gbs")], 4)
             if peaks else None,
             "launches_per_step": dom["launches"], "avg_launch_us": round(avg_ms * 1e3, 3),
             "avg_launch_us_source": "this run: the timed graph-replayed step apportioned by the launches' "

@@ -300,6 +300,8 @@ int   tlg_dev_copy(float *dst, const float *src, size_t n, void *stream);
  * reaches, sink[0]. */
 int   tlg_dev_read(const float *src, size_t n, float *sink, void *stream);
 int   tlg_dev_mfma_peak(float *out, int blocks, int iters, void *stream);
+/* The same with 32x32x16 bf16 MFMAs (32768 flop each). */
+int   tlg_dev_mfma_bf16_peak(float *out, int blocks, int iters, void *stream);
 /* Stream capture into a HIP graph: begin, enqueue work, end -> executable
  * graph handle; replay with tlg_graph_launch. */
 int   tlg_graph_begin(void *stream);

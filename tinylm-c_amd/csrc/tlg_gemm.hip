@@ -1236,6 +1236,36 @@ __global__ __launch_bounds__(256) void k_mfma_peak(float *__restrict__ out, int 
     out[(size_t)blockIdx.x * blockDim.x + threadIdx.x] = s;
 }
 
+// The same of the bf16 matrix cores, which the tiles use: v_mfma_f32_32x32x16_bf16.
+__global__ __launch_bounds__(256) void k_mfma_bf16_peak(float *__restrict__ out, int iters, float seed)
+{
+    f32x16 c0 = {}, c1 = {}, c2 = {}, c3 = {};
+    bf16x8 a, b;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        a[k] = (__bf16)(seed + k * 0.01f + threadIdx.x * 1e-3f);
+        b[k] = (__bf16)(seed - k * 0.01f - threadIdx.x * 1e-3f);
+    }
+    for (int i = 0; i < iters; i++) {
+        c0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c0, 0, 0, 0);
+        c1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c1, 0, 0, 0);
+        c2 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, a, c2, 0, 0, 0);
+        c3 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, b, c3, 0, 0, 0);
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; v++) s += c0[v] + c1[v] + c2[v] + c3[v];
+    out[(size_t)blockIdx.x * blockDim.x + threadIdx.x] = s;
+}
+
+int tlg_mfma_bf16_peak_launch(float *out, int blocks, int iters, hipStream_t st)
+{
+    if (blocks <= 0 || iters <= 0) return tlg_fail(TLG_EINVAL, "tlg_dev_mfma_bf16_peak: bad size");
+    hipLaunchKernelGGL(k_mfma_bf16_peak, dim3(blocks), dim3(256), 0, st, out, iters, 0.5f);
+    TLG_HIP(hipGetLastError());
+    return TLG_OK;
+}
+
 int tlg_mfma_peak_launch(float *out, int blocks, int iters, hipStream_t st)
 {
     if (blocks <= 0 || iters <= 0) return tlg_fail(TLG_EINVAL, "tlg_dev_mfma_peak: bad size");

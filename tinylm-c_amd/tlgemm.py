@@ -58,6 +58,7 @@ SIGNATURES = {
     "tlg_dev_copy": (_i, [_vp, _vp, _sz, _vp]),
     "tlg_dev_read": (_i, [_vp, _sz, _vp, _vp]),
     "tlg_dev_mfma_peak": (_i, [_vp, _i, _i, _vp]),
+    "tlg_dev_mfma_bf16_peak": (_i, [_vp, _i, _i, _vp]),
     "tlg_dev_gemm_group": (_i, [_vp, _i, _vp]),
     "tlg_dev_gemm_flush": (_i, [_vp]),
     "tlg_dev_gemm_pending": (_i, []),
