@@ -83,14 +83,14 @@ static GemmPlan make_plan(int ci, int Mo, int No, int R, int splits, size_t ws_f
 // Automatic choice: the largest of 128x128, 64x64 and 32x32 tiles that gives
 // the 256 CUs about 160 work items, splitting the reduction as far as every
 // split keeps >= 512 steps (small outputs with long reductions, i.e. mm_atb's
-// dW), 256 on 32x32 tiles (mm_atb (1001, 77, 333) 9.9 us in 3 splits, 13.6
-// whole).  Measured, best other shape against the rule's: mm (8192, 384, 2048)
-// 128x128 79 us, 128x64 83, 64x64 103; mm (4096, 768, 256) 64x64 14.5,
-// 32x32 20.2; mm (2048, 512, 128) 32x32 7.3, 64x64 10.7; mm_atb
-// (8192, 1024, 384) 8 splits of 128x128 47.5, 64x64 51.4.  64x64 tiles take
-// 64-step stages (8 waves, a quarter of each stage per wave) from 512 steps
-// on and 16-step stages below: 14.5 against 16.8 us at 768 steps, 7.5 against
-// 8.0 at 128.
+// dW), 256 on 32x32 tiles (mm_atb (1001, 77, 333) 11.3 us in 3 splits, 12.9
+// whole).  Measured on one box, other shapes against the rule's: mm
+// (8192, 384, 2048) 128x128 85 us, 64x64 97, 128x64 121; mm (4096, 768, 256)
+// 64x64 17, 32x32 23; mm (2048, 512, 128) 32x32 7.4, 64x64 11.4; mm_atb
+// (8192, 1024, 384) 7 splits of 128x128 52 (8 splits 47), 64x64 52.  64x64 tiles
+// take 64-step stages (8 waves, a quarter of each stage per wave) from 512 steps
+// on and 16-step stages below: 16.9 against 19.4 us at 768 steps, 19 against 11
+// at 128.
 //
 // Outputs of 240 64x64 tiles and more run whole: a split's partials lie in the
 // one workspace, which calls that overlap on two streams would both write, and
@@ -295,7 +295,7 @@ static int flush_foreign(hipStream_t st);
 // Tile shape of a grouped launch (all problems of a group share it): the
 // first row of kAuto whose shape gives the launch enough work items.  Measured
 // over the nano, m3 and m8 models' launches (replayed, us; the row's shape
-// against the next one's):
+// against the next one's; before operands were scaled, which took 1 to 2 %):
 //   128x128  m8 FFN backward 186 / 203 (128x64), m3 60 / 73; m8 W2 48 / 50.
 //            Launches without an mm_atb need whole rounds of 256 items (m8
 //            Q | K | V: 320 items, 35 against 32 on 64x64 tiles); short

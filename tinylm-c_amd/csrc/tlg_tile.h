@@ -12,23 +12,26 @@
 // waves form a WGM x WGN grid over the tile and WK groups along each stage of
 // BK reduction steps, each wave 32x32 blocks of it.
 //
-// The arithmetic: gfx950's matrix cores run bf16 at 16 times the fp32 rate
-// (measured 2.2 PFLOP/s against 146 TFLOP/s), so every fp32 operand is split,
-// exactly, into three bf16 pieces while it is staged, and a product into the
-// six piece products that reach 2^-25 of it: 367 TFLOP/s of fp32 work at that
+// The arithmetic: gfx950's matrix cores run bf16 at 14 times the fp32 rate
+// (k_mfma_bf16_peak 2.0 PFLOP/s, k_mfma_peak 146 TFLOP/s), so every fp32 operand
+// is split, exactly, into three bf16 pieces while it is staged, and a product into the
+// six piece products that reach 2^-25 of it: 336 TFLOP/s of fp32 work at that
 // rate.  Products of bf16 are exact in fp32 and a 32x32x16 MFMA rounds its
 // running sum once per 16 steps, so the result is closer to fp64's than the
 // fp32 MFMA chain's, which rounds at every step: 2.5 to 3 times, at 32 to 8192
 // steps (2.9e-7 -> 0.9e-7 at 256, 1.7e-6 -> 5.7e-7 at 8192, N(0, 1) values).
 //
-// What bounds it: matrix cores, vector instructions (13 per pair of values to
-// split), LDS (6 bytes per value written, then read by each wave that shares
-// it) and the loads all want more than half of a stage's cycles.  With reads,
-// splits and loads left out the 128x128 tile's MFMAs alone run at 319 TFLOP/s
-// at R = 1536; with them 190.  Loads run NR stages ahead into registers, the
-// split runs between the MFMAs, LDS is double buffered, one barrier per stage.
-// 8192 x 384 x 2048 (fwd / dX / dW) 117 / 152 / 157 -> 77 / 82 / 84 us against
-// the fp32 MFMA tiles this replaces; 4096 x 256 x 768 24 / 22 / 35 -> 14 / 17 / 23.
+// What bounds it: a stage's waits.  By counters (8192 x 384 x 2048, dX / fwd /
+// dW) the matrix cores are busy 40 / 41 / 38 % and the LDS 25 / 33 / 38 % of the
+// time, 0 / 16 / 37 % of the latter bank conflicts (operands along their output
+// index).  Beside them run the splits (13 vector instructions per pair of
+// values) and the loads, and one 8-wave workgroup a CU has nothing else to run
+// at a stage's barrier.  With reads, splits and loads left out the 128x128
+// tile's MFMAs alone ran at 319 TFLOP/s at R = 1536; with them 190.  Loads run
+// NR stages ahead into registers, the split runs between the MFMAs, LDS is
+// double buffered, one barrier per stage.
+// 8192 x 384 x 2048 (fwd / dX / dW) 117 / 152 / 157 -> 80 / 77 / 84 us against
+// the fp32 MFMA tiles this replaces; 4096 x 256 x 768 24 / 22 / 35 -> 14 / 16 / 21.
 //
 // Reduction order inside a 16-step MFMA: lanes 0-31 supply steps 0-7, lanes
 // 32-63 steps 8-15.  The result differs from the reference's sequential chain
@@ -354,11 +357,11 @@ struct Tile {
 };
 
 // Instruction order inside one stage's scheduling region (between two
-// barriers): the prefetch loads and every fragment read of the stage first,
-// then the MFMAs with the next stage's splits and LDS stores spread between
-// them.  An MFMA occupies the matrix core for 32 cycles and its wave's issue
-// for 4, so the ~14 vector instructions that split a float4 run under the
-// MFMAs instead of after them.
+// barriers): after the prefetch loads, behind each MFMA an even share of the
+// next stage's fragment reads, of the splits and of the LDS stores.  An MFMA
+// occupies the matrix core for 32 cycles and its wave's issue for 4, so the 26
+// vector instructions that split a float4 run under the MFMAs instead of after
+// them.
 template <int NM, int VALU, int DSW, int DSR, int I = 0>
 __device__ __forceinline__ void sched_mfmas()
 {
@@ -1363,9 +1366,8 @@ __global__ __launch_bounds__(T::THREADS) void k_group(GroupArgs g)
 // Every problem of such a launch shares one row-offset array; it is staged in
 // LDS once, so finding a work item's expert costs no dependent global loads.
 // The fused variants (gathered rows, paired columns, epilogues) are separate
-// inlined code paths; left alone the compiler gives their accumulators
-// disjoint AGPRs and the kernel drops to 3 waves per SIMD, so it is held to
-// the dense kernels' 4 (no spills at that bound).
+// inlined code paths that share one register allocation: two waves per SIMD
+// (64x64 tiles 171 VGPRs at four waves, 128x128 ones 245 at eight).
 #define TLG_MAX_EXPERTS 64
 template <class T>
 __global__ __launch_bounds__(T::THREADS) void k_expert_group(GroupArgs g)
