@@ -212,7 +212,7 @@ def test_gemv_group(lib):
 # before its MFMAs, out-of-range chunks loaded from a zero buffer) beside the
 # shapes they reorder
 SCHED_CFGS = [3, 24, 25, 14, 26, 20, 27, 22, 28, 13, 29, 15, 30, 0, 31, 1, 32, 8, 33, 11, 34, 21, 35, 23, 36, 18, 37,
-              38, 39, 40, 41, 42, 43, 44, 45, 46, 47, 48, 49, 50]
+              38, 39, 40, 41, 42, 43, 44, 45, 46, 47, 48, 49, 50, 9, 10, 12, 16, 17, 19]
 
 
 @pytest.mark.parametrize("gcfg", SCHED_CFGS)
@@ -546,6 +546,21 @@ def test_mm_bt_swiglu_bwd(lib, M, K, N):
     assert normwise_rel(u.cpu().numpy(), dact * z * sg) <= TOL
 
 
+@pytest.mark.parametrize("cfg", [9, 3, 14, 15])
+@pytest.mark.parametrize("shape", [(261, 132, 196), (129, 260, 324)], ids=str)
+def test_swiglu_on_every_shape(lib, cfg, shape):
+    """The fused SwiGLU launches on each tile shape of their automatic rule, where
+    rows, pairs of columns and stages end."""
+    M, K, N = shape
+    lib.check(lib.tlg_tune_expert(cfg, -1), "tune")
+    try:
+        test_swiglu_mm(lib, M, K, N)
+        test_mm_bt_swiglu_bwd(lib, M, K, N)
+    finally:
+        lib.check(lib.tlg_tune_expert(-1, -1), "tune")
+
+
+
 def test_fused_ffn_carries_pending_reduction(lib, orc):
     """A dense fused launch after a grouped launch with a split mm_atb: the
     deferred reduction rides along (or is flushed) and both results hold."""
@@ -646,7 +661,7 @@ def test_host_registry_device_residency(lib, orc):
     assert lib.tlg_mirror(buf.ctypes.data) is None
 
 
-@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4, 5, 6, 7, 8, 13, 14, 15])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15])
 def test_every_tile_config(lib, orc, cfg):
     """Each instantiated tile shape, with and without a split reduction, on a
     ragged shape (scalar staging) and an aligned one (float4 staging)."""
